@@ -9,6 +9,10 @@
 // with nothing visible averages every value, as mx.where + softmax do) or
 // offset by the additive mask, a softmax, and the weights times V.
 //
+// 16-bit queries with one head dim of 64, 96, 128 or 256 take the matrix-core
+// kernel of sdpa_stage.hip; this file's kernel serves fp32 queries and the
+// other head dims.
+//
 // Here everything after the inputs runs in fp32 (the reference rounds q*scale,
 // the scores and the weights to the query dtype in between; those roundings
 // are not restated). Kernel sdpa_gen_kernel: one workgroup per (query row,
@@ -28,40 +32,10 @@
 #include <algorithm>
 #include <cfloat>
 
-#include "common.h"
+#include "sdpa_gen.h"
 
 namespace sparkq {
 
-struct GenSdpaArgs {
-  const void* q;                  // [B,Hq,L,D] contiguous, q dtype
-  const uint32_t* kp;             // packed codes, D*bits/32 words per token
-  const void* ks;                 // scales [.., D/G], q dtype
-  const void* kb;                 // biases, same strides as scales
-  const uint32_t* vp;
-  const void* vs;
-  const void* vb;
-  const void* mask;               // mask array or null
-  void* out;                      // [B,Hq,L,Dv]
-  float* pm;                      // split partials: max [rows][S]
-  float* pz;                      //   sums [rows][S]
-  float* pacc;                    //   outputs [rows][S][Dv]
-  int64_t kp_b, kp_h, kp_t;       // strides in words
-  int64_t ks_b, ks_h, ks_t;       // strides in elements (biases share them)
-  int64_t vp_b, vp_h, vp_t;
-  int64_t vs_b, vs_h, vs_t;
-  int64_t m_b, m_h, m_l, m_n;     // mask strides in elements (0 to broadcast)
-  int mask_kind;                  // kMask*
-  int mask_dtype;                 // additive masks: SPARKQ_F32/F16/BF16
-  int B, Hq, Hkv, L, N, D, Dv, G, bits;
-  int q_dtype, out_dtype;
-  int RC, nch;                    // query heads per workgroup, chunks per KV head
-  int S, tps;                     // context splits, tokens per split
-  int vt;                         // value tokens per LDS stage
-  float scale_log2;               // softmax scale times log2(e)
-  float masked;                   // score of a masked entry, in log2 units
-};
-
-[[maybe_unused]] constexpr int kMaskNone = 0, kMaskCausal = 1, kMaskBool = 2, kMaskAdd = 3;
 constexpr int kGenMaxRC = 8;
 constexpr int kGenMaxDim = 512;
 constexpr int kGenChunk = 256;
@@ -407,15 +381,22 @@ static void launch_gen_b(const GenSdpaArgs& a, int bits, bool mf32, dim3 grid, s
     launch_gen_m<8>(a, mf32, grid, lds, st);
 }
 
+// bytes of S splits' partials: maxima, sums, outputs
+static size_t gen_partial_bytes(size_t rows, int64_t S, int64_t Dv) {
+  if (S <= 1) return 0;
+  return round_up(rows * S * 4, 256) * 2 + round_up(rows * S * Dv * 4, 256);
+}
+
+// covers both kernels (the query type and the key head dim, which choose
+// between them, are not known here)
 size_t sdpa_gen_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
                           int64_t Dv) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || N <= 0 || Dv <= 0 || Hq % Hkv) return 0;
   int RC, nch, S;
   int64_t tps;
   gen_plan(B, Hq, Hkv, L, N, &RC, &nch, &S, &tps);
-  if (S == 1) return 0;
   const size_t rows = (size_t)B * Hq * L;
-  return round_up(rows * S * 4, 256) * 2 + round_up(rows * S * Dv * 4, 256);
+  return gen_partial_bytes(rows, std::max(S, sdpa_stage_splits(B, Hq, Hkv, L, N)), Dv);
 }
 
 int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, const void* vp,
@@ -468,6 +449,8 @@ int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, 
   int64_t tps;
   gen_plan(B, Hq, Hkv, L, N, &a.RC, &a.nch, &a.S, &tps);
   a.tps = (int)tps;
+  const bool stage = sdpa_stage_ok(a);
+  if (stage) a.S = sdpa_stage_splits(B, Hq, Hkv, L, N);
   a.scale_log2 = scale * 1.4426950408889634f;
   // the reference fills masked scores with the lowest finite value of the
   // query dtype: any visible score outweighs it completely, and a row with
@@ -477,7 +460,7 @@ int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, 
   a.masked = qdt == SPARKQ_F16 ? -65504.0f : qdt == SPARKQ_BF16 ? -3.38953139e38f
                                                                   : -3.40282347e38f;
   if (a.S > 1) {
-    const size_t need = sdpa_gen_workspace(B, Hq, Hkv, L, N, Dv);
+    const size_t need = gen_partial_bytes((size_t)B * Hq * L, a.S, Dv);
     if (ws == nullptr || wsb < need)
       return set_error(SPARKQ_ERR_WORKSPACE,
                        "quantized_sdpa needs a workspace of %zu bytes (got %zu)", need, wsb);
@@ -487,11 +470,15 @@ int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, 
     a.pz = reinterpret_cast<float*>(p + round_up(rows * a.S * 4, 256));
     a.pacc = reinterpret_cast<float*>(p + 2 * round_up(rows * a.S * 4, 256));
   }
-  a.vt = gen_value_tokens(a.RC, (int)D, (int)Dv);
-  const size_t lds = gen_lds_bytes(a.RC, (int)D, (int)Dv);
-  const dim3 grid((unsigned)(L * a.S), (unsigned)(B * Hkv * a.nch));
-  launch_gen_b(a, bits, qdt == SPARKQ_F32, grid, lds, st);
-  if (int rc = check_launch("sdpa_gen_kernel")) return rc;
+  if (stage) {
+    if (int rc = launch_sdpa_stage(a, st)) return rc;
+  } else {
+    a.vt = gen_value_tokens(a.RC, (int)D, (int)Dv);
+    const size_t lds = gen_lds_bytes(a.RC, (int)D, (int)Dv);
+    const dim3 grid((unsigned)(L * a.S), (unsigned)(B * Hkv * a.nch));
+    launch_gen_b(a, bits, qdt == SPARKQ_F32, grid, lds, st);
+    if (int rc = check_launch("sdpa_gen_kernel")) return rc;
+  }
   if (a.S > 1) {
     hipLaunchKernelGGL(sdpa_gen_merge_kernel, dim3((unsigned)(B * Hq * L)), dim3(256), 0, st,
                        a.pm, a.pz, a.pacc, out, odt, a.S, (int)Dv);
