@@ -312,21 +312,31 @@ __device__ __forceinline__ float erf_for16(float t) {
   return e;
 }
 
+// v rounded to T and back: the low half of the packed conversion (one
+// instruction for bf16, against six of the bit-level rounding)
+template <typename T>
+__device__ __forceinline__ float round16(float v) {
+  return lo16<T>(pack_round<T>(v, 0.0f));
+}
+
 // gelu(gate) * up as mlx.nn.gelu computes it on a 16-bit array,
 // x * (1 + erf(x / sqrt(2))) / 2 (spark_mlx_llm/ops/ffn.py:102): the constant
 // sqrt(2) is rounded to T (1.4140625 for both types) and each operation's
 // result is rounded to T. erf runs in double and is rounded to fp32 first,
 // as a float erf would deliver it. g and u are the projections' fp32 sums;
 // the result is the product's fp32 value, which the caller rounds to T.
+//
+// The division by 1.4140625 = 181/128 is a product with its fp32 reciprocal:
+// a quotient 128 gate / 181 of an 11-bit gate lies at least 1/181 of half a
+// unit of T from a rounding tie (181 is prime, so none is exact), far more
+// than the product's two fp32 roundings, and rounds to the same T.
 template <typename T>
 __device__ __forceinline__ float gelu_mul(float g, float u) {
-  auto r = [](float v) { return T::to_f32(T::from_f32(v)); };
-  const float gate = r(g), up = r(u);
-  const float c = r(1.41421356237309515f);
-  const float t1 = r(gate / c);
-  const float e = r(erf_for16<T>(t1));
-  const float t3 = r(1.0f + e);
-  const float t5 = r(r(gate * t3) / 2.0f);
+  const float gate = round16<T>(g), up = round16<T>(u);
+  const float t1 = round16<T>(gate * (1.0f / 1.4140625f));
+  const float e = round16<T>(erf_for16<T>(t1));
+  const float t3 = round16<T>(1.0f + e);
+  const float t5 = round16<T>(round16<T>(gate * t3) * 0.5f);
   return t5 * up;
 }
 

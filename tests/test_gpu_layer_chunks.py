@@ -1,0 +1,62 @@
+"""GPU parity of the 16-byte forms of the layer's elementwise kernels where
+they begin and end: RMSNorm rows around the chunk counts it is built for, rows
+and tensors it leaves to the element-by-element form, and the FFN's gelu * up
+over partial and several workgroups."""
+
+import numpy as np
+import pytest
+import torch
+
+import oracle as o
+from helpers import down16, ulp_distance16, up16
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("k", [8, 100, 2048, 2056, 2560, 4096, 4104, 8192, 8200])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_rms_norm_chunks(gpu, k, offset):
+    """A mean square summed in fp32 in any order moves a row's norm by a few
+    fp32 units: at most one unit of the 16-bit result, in few elements."""
+    import sparkq
+
+    m = 3
+    print(f"[case] rms_norm k={k} offset={offset}", flush=True)
+    for dtype in (o.BF16, o.F16):
+        x = o.randn16(k, 1, m * k, 1.0, dtype).reshape(m, k)
+        r = o.randn16(k, 2, m * k, 1.0, dtype).reshape(m, k)
+        w = o.round16(1.0 + 0.2 * o.randn(k, 3, k), dtype)
+
+        def place(a):
+            t = up16(a, dtype, gpu)
+            flat = torch.empty(t.numel() + offset, dtype=t.dtype, device=gpu)[offset:]
+            return flat.copy_(t.reshape(-1)).view(t.shape)
+
+        for res in (None, r):
+            h = x if res is None else o.add16(x, r, dtype)
+            n = sparkq.rms_norm(place(x), place(w), 1e-5,
+                                residual=None if res is None else place(r))
+            d = ulp_distance16(down16(n), o.rms_norm16(h, w, 1e-5, dtype), dtype)
+            assert d.max() <= 1 and (d == 0).mean() > 0.98
+
+
+@pytest.mark.parametrize("m,inter", [(5, 64), (33, 2112), (40, 128)])
+def test_gelu_chunks(gpu, m, inter):
+    """act of the composed FFN equals the oracle's gelu(gate) * up of the
+    device's own projections, bit for bit."""
+    import sparkq
+    from test_gpu_layer import _dev, _mat, _plain
+
+    k, g = 64, 32
+    print(f"[case] gelu m={m} I={inter}", flush=True)
+    for dtype in (o.BF16, o.F16):
+        x = o.randn16(m, 1, m * k, 3.0, dtype).reshape(m, k)
+        nw = o.round16(np.ones(k, np.float32), dtype)
+        gate, up = (_mat(m, s, inter, k, g, dtype) for s in (4, 5))
+        down = _mat(m, 6, k, inter, g, dtype)
+        _, _, nrm, act = (down16(t) for t in sparkq.fused_ffn(
+            up16(x, dtype, gpu), up16(0 * x, dtype, gpu), up16(nw, dtype, gpu), 1e-6,
+            _dev(gate, gpu, dtype), _dev(up, gpu, dtype), _dev(down, gpu, dtype), group_size=g,
+            return_intermediates=True))
+        g16, u16 = (_plain(nrm, t, g, dtype, gpu) for t in (gate, up))
+        assert np.array_equal(act, o.gelu_mul16(g16, u16, dtype))
