@@ -257,6 +257,15 @@ int sparkq_w8_affine_linear(const void* x, const uint32_t* w, const void* scales
                             int group_size, int x_dtype, int scale_dtype, int y_dtype,
                             void* stream);
 
+/* The same with a workspace (256-byte aligned, at least
+ * sparkq_w8_affine_workspace_bytes, which may be 0; null runs the kernel that
+ * needs none): K is then split over the chip. */
+size_t sparkq_w8_affine_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_size);
+int sparkq_w8_affine_linear_ws(const void* x, const uint32_t* w, const void* scales,
+                               const void* biases, void* y, int64_t M, int64_t N, int64_t K,
+                               int group_size, int x_dtype, int scale_dtype, int y_dtype,
+                               void* workspace, size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * INT8-KV GQA decode attention (one query token per sequence)
  *   q    [B,Hq,D] (the L=1 axis of [B,Hq,1,D] dropped), q_dtype

@@ -69,8 +69,9 @@ int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, co
 int w8a16_linear(const void* x, const int8_t* w, const float* scales, void* y, int64_t M,
                  int64_t N, int64_t K, int xdt, int ydt, hipStream_t st);
 int w8_affine_linear(const void* x, const uint32_t* w, const void* s, const void* b, void* y,
-                     int64_t M, int64_t N, int64_t K, int G, int xdt, int sdt, int ydt,
-                     hipStream_t st);
+                     int64_t M, int64_t N, int64_t K, int G, int xdt, int sdt, int ydt, void* ws,
+                     size_t wsb, hipStream_t st);
+size_t w8_affine_workspace(int64_t M, int64_t N, int64_t K, int G);
 // launchers (layer.hip)
 size_t ffn_workspace(int64_t M, int64_t K, int64_t I, int G);
 int ffn(const void* x, const void* attn, const void* nw, float eps, const uint32_t* wg,
@@ -609,10 +610,24 @@ int sparkq_w8a16_linear(const void* x, const int8_t* w, const float* scales, voi
   return w8a16_linear(x, w, scales, y, M, N, K, x_dtype, y_dtype, (hipStream_t)stream);
 }
 
+size_t sparkq_w8_affine_workspace_bytes(int64_t M, int64_t N, int64_t K, int group_size) {
+  if (M <= 0 || N <= 0 || K <= 0 || (group_size != 32 && group_size != 64 && group_size != 128))
+    return 0;
+  return w8_affine_workspace(M, N, K, group_size);
+}
+
 int sparkq_w8_affine_linear(const void* x, const uint32_t* w, const void* scales,
                             const void* biases, void* y, int64_t M, int64_t N, int64_t K,
                             int group_size, int x_dtype, int scale_dtype, int y_dtype,
                             void* stream) {
+  return sparkq_w8_affine_linear_ws(x, w, scales, biases, y, M, N, K, group_size, x_dtype,
+                                    scale_dtype, y_dtype, nullptr, 0, stream);
+}
+
+int sparkq_w8_affine_linear_ws(const void* x, const uint32_t* w, const void* scales,
+                               const void* biases, void* y, int64_t M, int64_t N, int64_t K,
+                               int group_size, int x_dtype, int scale_dtype, int y_dtype,
+                               void* workspace, size_t workspace_bytes, void* stream) {
   REQUIRE(x && w && scales && biases && y, "w8_affine_linear: null tensor pointer");
   REQUIRE(M > 0 && N > 0 && K > 0, "w8_affine_linear: M, N and K must be positive");
   REQUIRE(M <= kI32Max && N <= kI32Max && K <= kI32Max, "w8_affine_linear: dimension too large");
@@ -628,11 +643,12 @@ int sparkq_w8_affine_linear(const void* x, const uint32_t* w, const void* scales
                     "w8_affine_linear: weights or activations exceed the 2 GiB range of one "
                     "buffer descriptor");
   REQUIRE(aligned(x, 16) && aligned(w, 16), "w8_affine_linear: x and w must be 16-byte aligned");
+  REQUIRE(aligned(workspace, 256), "w8_affine_linear: the workspace must be 256-byte aligned");
   REQUIRE(aligned(scales, 2) && aligned(biases, 2) && aligned(y, 4),
           "w8_affine_linear: scales, biases and y must be aligned to their element size");
   DEVICE_OK();
   return w8_affine_linear(x, w, scales, biases, y, M, N, K, group_size, x_dtype, scale_dtype,
-                          y_dtype, (hipStream_t)stream);
+                          y_dtype, workspace, workspace_bytes, (hipStream_t)stream);
 }
 
 size_t sparkq_ffn_workspace_bytes(int64_t M, int64_t K, int64_t I, int group_size) {

@@ -34,9 +34,7 @@
 //                       through LDS), fp16 MFMA 32x32x16 with no per-group
 //                       epilogue, the bias slots on the bf16 MFMA, split-K
 //                       combined in the same launch when tiles are few
-//   xsum_kernel         group sums X_g[m] for the fp16 GEMM, layout [K/G][M]
-//   w4_gemm_kernel      fp16, M > 32: 128x128x64 LDS tiles (B decoded to the
-//                       exact q), per-group fp32 scale and bias epilogue
+// float16 activations from 33 rows take the prefill kernel of affgemm.hip.
 #include <algorithm>
 #include <type_traits>
 #include <cmath>
@@ -1647,34 +1645,7 @@ __global__ __launch_bounds__(256, 2) void w4_skinny_kernel(SkinnyArgs a) {
 // ---------------------------------------------------------------------------
 // GEMM (M > 32)
 // ---------------------------------------------------------------------------
-// group sums X_g[m] in fp32, stored [K/G][M]; one thread per (m, g)
-template <typename T>
-__global__ __launch_bounds__(256) void xsum_kernel(const uint16_t* __restrict__ x,
-                                                   float* __restrict__ xsum,
-                                                   int M, int K, int G) {
-  const int ng = K / G;
-  const int64_t id = (int64_t)blockIdx.x * 256 + threadIdx.x;
-  if (id >= (int64_t)M * ng) return;
-  const int m = (int)(id / ng), g = (int)(id - (int64_t)m * ng);
-  const u32x4_t* src = reinterpret_cast<const u32x4_t*>(x + (int64_t)m * K + (int64_t)g * G);
-  float s = 0.0f;
-  for (int i = 0; i < G / 8; ++i) {
-    const u32x4_t v = src[i];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      s += T::to_f32((uint16_t)(v[e] & 0xFFFFu));
-      s += T::to_f32((uint16_t)(v[e] >> 16));
-    }
-  }
-  xsum[(int64_t)g * M + m] = s;
-}
-
-constexpr int kBM = 128, kBN = 128, kBK = 64;
-
-// element offset of the 16-byte piece (row, kc) in a swizzled [128][64] tile
-__device__ __forceinline__ int tile_off(int row, int kc) {
-  return row * 64 + ((kc ^ (row & 7)) << 3);
-}
+constexpr int kBK = 64;
 
 // ---------------------------------------------------------------------------
 // bf16 prefill GEMM on exact fp16 operands
@@ -2317,154 +2288,6 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
     }
 }
 
-template <typename T, int G>
-__global__ __launch_bounds__(256, 2) void w4_gemm_kernel(
-    const uint16_t* __restrict__ x, const uint32_t* __restrict__ w,
-    const uint16_t* __restrict__ sc, const uint16_t* __restrict__ bi,
-    const float* __restrict__ xsum, void* __restrict__ y, int y_dtype, int M,
-    int N, int K) {
-  constexpr int GPS = G == 32 ? 2 : 1;  // groups starting inside one k-step
-  __shared__ __attribute__((aligned(16))) uint16_t As[2][kBM * kBK];
-  __shared__ __attribute__((aligned(16))) uint16_t Bs[2][kBN * kBK];
-  __shared__ __attribute__((aligned(16))) float SBs[2][GPS][kBN][2];
-  __shared__ __attribute__((aligned(16))) float XSs[2][GPS][kBM];
-
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int j = lane >> 5;
-  const int wm = wave & 1, wn = wave >> 1;
-  const int n0 = blockIdx.x * kBN, m0 = blockIdx.y * kBM;
-  const int ngroups = K / G;
-  const int nsteps = K / kBK;
-
-  const DecodeConsts dc = decode_consts<T>();
-  // global -> register staging
-  u32x4_t ra[4], rb;
-  float rs = 0.0f, rbias = 0.0f, rx = 0.0f;
-
-  auto load = [&](int step) {
-    const int k0 = step * kBK;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int p = tid + 256 * i, row = p >> 3, kc = p & 7;
-      const int gm = m0 + row;
-      ra[i] = u32x4_t{0u, 0u, 0u, 0u};
-      if (gm < M) ra[i] = *reinterpret_cast<const u32x4_t*>(x + (int64_t)gm * K + k0 + kc * 8);
-    }
-    {
-      const int row = tid >> 1, half = tid & 1, gn = n0 + row;
-      rb = u32x4_t{0u, 0u, 0u, 0u};
-      if (gn < N) rb = *reinterpret_cast<const u32x4_t*>(w + (int64_t)gn * (K >> 3) + (k0 >> 3) + 4 * half);
-    }
-    if (tid < 128 * GPS) {
-      const int gi = tid >> 7, row = tid & 127;
-      const int g = (G == 32) ? 2 * step + gi : (k0 / G);
-      const int gn = n0 + row, gm = m0 + row;
-      rs = 0.0f;
-      rbias = 0.0f;
-      rx = 0.0f;
-      if (gn < N) {
-        rs = T::to_f32(sc[(int64_t)gn * ngroups + g]);
-        rbias = T::to_f32(bi[(int64_t)gn * ngroups + g]);
-      }
-      if (gm < M) rx = xsum[(int64_t)g * M + gm];
-    }
-  };
-  auto store = [&](int st) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int p = tid + 256 * i, row = p >> 3, kc = p & 7;
-      *reinterpret_cast<u32x4_t*>(&As[st][tile_off(row, kc)]) = ra[i];
-    }
-    {
-      const int row = tid >> 1, half = tid & 1;
-#pragma unroll
-      for (int wi = 0; wi < 4; ++wi)
-        *reinterpret_cast<u32x4_t*>(&Bs[st][tile_off(row, 4 * half + wi)]) = decode_w4<T>(rb[wi], dc);
-    }
-    if (tid < 128 * GPS) {
-      const int gi = tid >> 7, row = tid & 127;
-      SBs[st][gi][row][0] = rs;
-      SBs[st][gi][row][1] = fmaf(-T::OFFSET, rs, rbias);
-      XSs[st][gi][row] = rx;
-    }
-  };
-
-  f32x16_t acc[2][2], tmp[2][2];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      acc[a][b] = f32x16_t{};
-      tmp[a][b] = f32x16_t{};
-    }
-
-  load(0);
-  store(0);
-  __syncthreads();
-
-  for (int step = 0; step < nsteps; ++step) {
-    const int st = step & 1;
-    if (step + 1 < nsteps) load(step + 1);
-#pragma unroll
-    for (int ss = 0; ss < 4; ++ss) {
-      const int kc = 2 * ss + j;
-      u32x4_t af[2], bf[2];
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const int ar = wm * 64 + t * 32 + (lane & 31);
-        const int br = wn * 64 + t * 32 + (lane & 31);
-        af[t] = *reinterpret_cast<const u32x4_t*>(&As[st][tile_off(ar, kc)]);
-        bf[t] = *reinterpret_cast<const u32x4_t*>(&Bs[st][tile_off(br, kc)]);
-      }
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b) tmp[a][b] = mfma32x32x16<T>(af[a], bf[b], tmp[a][b]);
-
-      const bool group_end =
-          (G == 32) ? (ss == 1 || ss == 3) : (G == 64 ? ss == 3 : (ss == 3 && (step & 1)));
-      if (group_end) {
-        const int gi = (G == 32) ? (ss >> 1) : 0;
-#pragma unroll
-        for (int b = 0; b < 2; ++b) {
-          const int br = wn * 64 + b * 32 + (lane & 31);
-          const float s = SBs[st][gi][br][0], bp = SBs[st][gi][br][1];
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-#pragma unroll
-            for (int q4 = 0; q4 < 4; ++q4) {
-              const int mr = wm * 64 + a * 32 + 8 * q4 + 4 * j;
-              const f32x4_t xv = *reinterpret_cast<const f32x4_t*>(&XSs[st][gi][mr]);
-#pragma unroll
-              for (int r = 0; r < 4; ++r) {
-                const int v = 4 * q4 + r;
-                const float t = fmaf(s, tmp[a][b][v], acc[a][b][v]);
-                acc[a][b][v] = fmaf(bp, xv[r], t);
-              }
-            }
-            tmp[a][b] = f32x16_t{};
-          }
-        }
-      }
-    }
-    if (step + 1 < nsteps) store(st ^ 1);
-    __syncthreads();
-  }
-
-  // epilogue
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const int gn = n0 + wn * 64 + b * 32 + (lane & 31);
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const int gm = m0 + wm * 64 + a * 32 + mfma32_row(lane, v);
-        if (gm < M && gn < N) store_out(y, (int64_t)gm * N + gn, acc[a][b][v], y_dtype);
-      }
-    }
-}
-
 // ---------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------
@@ -3080,6 +2903,12 @@ static WidePlan plan_wide(int64_t M, int64_t N, int64_t K) {
   return p;
 }
 
+// float16 activations from 33 rows (affgemm.hip)
+size_t affine_gemm_workspace(int64_t M, int64_t N, int64_t K, int G);
+int affine_gemm(const void* x, const uint32_t* w, const void* s, const void* b, void* y, int64_t M,
+                int64_t N, int64_t K, int G, int bits, int xdt, int sdt, int ydt,
+                unsigned char* ws, hipStream_t st);
+
 int64_t w4_mr_workspace(int64_t M, int64_t N, int64_t K, int G);
 int w4_mr_linear(const void* x, const uint32_t* w, const void* s, const void* b, void* y,
                  int64_t M, int64_t N, int64_t K, int G, int xdt, int ydt, hipStream_t st,
@@ -3099,8 +2928,8 @@ size_t w4a16_workspace(int64_t M, int64_t N, int64_t K, int G) {
     return p.S > 1 ? kCounterBytes + p.part_bytes : 0;
   }
   const GemmX16Layout l = gemm_x16_layout(M, N, K, G);
-  return kCounterBytes +
-         std::max(round_up((size_t)(K / G) * M * 4, 256), l.bytes + plan_wide(M, N, K).part_bytes);
+  return kCounterBytes + std::max(affine_gemm_workspace(M, N, K, G),
+                                  l.bytes + plan_wide(M, N, K).part_bytes);
 }
 
 template <typename T, int G, int MB, int CPW>
@@ -3138,26 +2967,6 @@ static void launch_skinny(const SkinnyPlan& p, int G, const SkinnyArgs& a, hipSt
     launch_skinny_g<T, 64>(p, a, st);
   else
     launch_skinny_g<T, 128>(p, a, st);
-}
-
-template <typename T>
-static void launch_gemm(int G, const void* x, const uint32_t* w, const void* s,
-                        const void* b, float* xs, void* y, int ydt, int M, int N,
-                        int K, hipStream_t st) {
-  const int64_t nxs = (int64_t)M * (K / G);
-  hipLaunchKernelGGL(xsum_kernel<T>, dim3((unsigned)cdiv(nxs, 256)), dim3(256), 0, st,
-                     (const uint16_t*)x, xs, M, K, G);
-  dim3 grid((unsigned)cdiv(N, kBN), (unsigned)cdiv(M, kBM));
-#define SPARKQ_GEMM(GG)                                                              \
-  hipLaunchKernelGGL((w4_gemm_kernel<T, GG>), grid, dim3(256), 0, st, (const uint16_t*)x, \
-                     w, (const uint16_t*)s, (const uint16_t*)b, xs, y, ydt, M, N, K)
-  if (G == 32)
-    SPARKQ_GEMM(32);
-  else if (G == 64)
-    SPARKQ_GEMM(64);
-  else
-    SPARKQ_GEMM(128);
-#undef SPARKQ_GEMM
 }
 
 // One launch of the prologue over M activation rows and the weight rows of
@@ -3418,18 +3227,13 @@ int w4a16_linear(const void* x, const uint32_t* w, const void* s, const void* b,
     return check_launch("w4_skinny_kernel");
   }
   unsigned char* wsp = reinterpret_cast<unsigned char*>(ws) + kCounterBytes;
-  if (xdt == SPARKQ_BF16 && !env_int("SPARKQ_W4_NO_X16", 0)) {
+  if (xdt == SPARKQ_BF16) {
     launch_gemm_x16(G, x, w, s, b, reinterpret_cast<const unsigned char*>(prep),
                     reinterpret_cast<unsigned*>(ws), wsp, y, ydt, (int)M, (int)N,
                     (int)K, st);
     return check_launch("w4_gemm_x16w_kernel");
   }
-  float* xs = reinterpret_cast<float*>(wsp);
-  if (xdt == SPARKQ_BF16)
-    launch_gemm<BF16>(G, x, w, s, b, xs, y, ydt, (int)M, (int)N, (int)K, st);
-  else
-    launch_gemm<F16>(G, x, w, s, b, xs, y, ydt, (int)M, (int)N, (int)K, st);
-  return check_launch("w4_gemm_kernel");
+  return affine_gemm(x, w, s, b, y, M, N, K, G, 4, xdt, xdt, ydt, wsp, st);
 }
 
 size_t w4a16_prepared_bytes(int64_t N, int64_t K, int G) {

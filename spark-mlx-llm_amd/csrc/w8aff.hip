@@ -8,7 +8,8 @@
 // affine nn.QuantizedLinear for prefill and verify rows, and 'native'/'auto'
 // W8 checkpoints use it for every input, :651-711).
 //
-// Kernel w8_affine_kernel. A workgroup of 4 waves owns a 32 x 128 output
+// Kernel w8_affine_kernel (calls without a workspace; with one, affgemm.hip).
+// A workgroup of 4 waves owns a 32 x 128 output
 // tile, each wave 32 activation rows x 32 weight rows as 2 x 2 blocks of the
 // 16x16x32 MFMA:
 //  * every code 0..255 is an exact 16-bit operand (bf16 and fp16 hold 8
@@ -205,9 +206,34 @@ __global__ __launch_bounds__(256) void w8_affine_kernel(W8AffArgs a, int G) {
     }
 }
 
+// affgemm.hip
+size_t affine_gemm_workspace(int64_t M, int64_t N, int64_t K, int G);
+int affine_gemm(const void* x, const uint32_t* w, const void* s, const void* b, void* y, int64_t M,
+                int64_t N, int64_t K, int G, int bits, int xdt, int sdt, int ydt,
+                unsigned char* ws, hipStream_t st);
+
+// Given a workspace, the kernels of affgemm.hip take the call from one row on:
+// they split K over the chip, where the kernel here walks it in one chain
+// (bf16, us per call, here -> there: 1 row of 3584 x 2560 G64 54 -> 18, of
+// 2560 x 4096 G32 182 -> 21, of 131072 x 2560 216 -> 136; 32 rows 66 -> 19,
+// 200 -> 22, 281 -> 142). The kernel here serves calls without a workspace.
+static bool w8_affine_gemm(int64_t M) { return M >= env_int("SPARKQ_W8AFF_GEMM_FROM", 1); }
+
+size_t w8_affine_workspace(int64_t M, int64_t N, int64_t K, int G) {
+  return w8_affine_gemm(M) ? affine_gemm_workspace(M, N, K, G) : 0;
+}
+
 int w8_affine_linear(const void* x, const uint32_t* w, const void* s, const void* b, void* y,
-                     int64_t M, int64_t N, int64_t K, int G, int xdt, int sdt, int ydt,
-                     hipStream_t st) {
+                     int64_t M, int64_t N, int64_t K, int G, int xdt, int sdt, int ydt, void* ws,
+                     size_t wsb, hipStream_t st) {
+  if (ws != nullptr && w8_affine_gemm(M)) {
+    const size_t need = w8_affine_workspace(M, N, K, G);
+    if (wsb < need)
+      return set_error(SPARKQ_ERR_WORKSPACE,
+                       "w8_affine_linear needs a workspace of %zu bytes (got %zu)", need, wsb);
+    return affine_gemm(x, w, s, b, y, M, N, K, G, 8, xdt, sdt, ydt,
+                       reinterpret_cast<unsigned char*>(ws), st);
+  }
   W8AffArgs a{};
   a.x = (const uint16_t*)x;
   a.w = w;

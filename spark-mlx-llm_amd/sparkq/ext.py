@@ -240,9 +240,11 @@ def _w8_affine_matmul(op, x, weight, scales, biases, group_size, out_dtype, out)
         return y.reshape(*lead, n)
     x2 = x.reshape(m, k).contiguous()
     weight, scales, biases = weight.contiguous(), scales.contiguous(), biases.contiguous()
-    _lib.call("sparkq_w8_affine_linear", _ptr(x2), _ptr(weight), _ptr(scales), _ptr(biases),
+    ws, wsb = _lib.workspace(x.device, _lib.lib().sparkq_w8_affine_workspace_bytes(
+        m, n, k, group_size), "w8_affine")
+    _lib.call("sparkq_w8_affine_linear_ws", _ptr(x2), _ptr(weight), _ptr(scales), _ptr(biases),
               _ptr(y), m, n, k, group_size, _lib.dtype_code(x.dtype),
-              _lib.dtype_code(scales.dtype), _lib.dtype_code(out_dtype),
+              _lib.dtype_code(scales.dtype), _lib.dtype_code(out_dtype), ws, wsb,
               _lib.stream_handle(x.device), device=x.device)
     return y.reshape(*lead, n)
 
