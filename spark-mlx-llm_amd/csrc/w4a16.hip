@@ -1681,7 +1681,7 @@ struct GemmPrepArgs {
   uint16_t* xh;        // [M][K] fp16, scaled and chunk-permuted
   int* ex;             // [M]
   uint16_t* a2;        // [M][K2p] bf16
-  uint16_t* sp;        // [N][K/G] fp16 scaled scales
+  uint16_t* sp;        // [K/G][N] fp16 scaled scales (a wave's columns side by side)
   int* es;             // [N]
   uint16_t* b2;        // [N][K2p] bf16
   int M, N, K, G, K2p;
@@ -1840,14 +1840,14 @@ __global__ __launch_bounds__(256) void gemm_prep_kernel(GemmPrepArgs a) {
   }
   // rw <= 64 rows: the four threads of a row are the threads above
   __syncthreads();
-  uint16_t* spr = a.sp + (int64_t)n0 * ng;
   uint16_t* sl16 = reinterpret_cast<uint16_t*>(slots);
   const int K2p = a.K2p;
-  for (int i = tid; i < nel; i += 256) {
-    const int r = i / ng, g = i - r * ng;
-    const uint32_t pv = pair[i];
+  for (int i = tid; i < ng * rw; i += 256) {  // rows fastest: the scales' store order
+    const int g = i / rw, r = i - g * rw;
+    if (r >= nr) continue;
+    const uint32_t pv = pair[r * ng + g];
     const float sf = bf16_to_f32((uint16_t)pv);
-    spr[i] = f32_to_f16(ldexpf(sf, -rexp[r]));
+    a.sp[(int64_t)g * a.N + n0 + r] = f32_to_f16(ldexpf(sf, -rexp[r]));
     uint16_t hi, lo;
     split_bf16(fmaf(8.0f, sf, bf16_to_f32((uint16_t)(pv >> 16))), hi, lo);
     sl16[r * K2p + 3 * g] = hi;
@@ -1886,7 +1886,7 @@ static PrepPlan plan_prep(int K, int G) {
 struct GemmX16Args {
   const uint16_t* xh;  // [M][K] fp16 from the prologue
   const uint32_t* w;   // [N][K/8]
-  const uint16_t* sp;  // [N][K/G] fp16
+  const uint16_t* sp;  // [K/G][N] fp16
   const int* ex;       // [M]
   const int* es;       // [N]
   const uint16_t* a2;  // [M][K2p]
@@ -1936,6 +1936,14 @@ __device__ __forceinline__ uint32_t bf16x2_rne(float lo, float hi) {
   return __builtin_bit_cast(uint32_t, v);
 }
 
+// The scales come in [K/G][N] order, so that a wave's 64 columns share a line
+// (in the checkpoint's order each lane's two bytes took a line of their own at
+// every step), and the serial tails keep several loads in flight: the bias
+// slots two to four sixteens, the pieces' sums whole batches of accumulators.
+// Per call without prepared weights, before -> now: down 2560 x 9728 M = 512
+// 72 -> 66 us, M = 1000 111 -> 96; gate 9728 x 2560 M = 1000 81 -> 78; QKV
+// 3584 x 2560 M = 64 37 -> 34; gate+up 19456 x 2560 M = 2048 232 -> 224.
+//
 // PD: 1 = the loads of step s+1 go out during step s, 2 = those of step s+2.
 // SCH (schedule variants, PD = 1): bit 0 raises the wave priority over the
 // MFMA phase of each step; bit 1 keeps four A slots in LDS, fills slot s+2
@@ -1984,7 +1992,8 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
   // rows past the tile's last one read as zero
   const rsrc_t rx = make_rsrc(a.xh + (int64_t)m0 * K, (uint32_t)mrows * (uint32_t)K * 2u);
   const rsrc_t rw = make_rsrc(a.w + (int64_t)wn0 * (K / 8), (uint32_t)nrows * (uint32_t)K / 2u);
-  const rsrc_t rs = make_rsrc(a.sp + (int64_t)wn0 * ng, (uint32_t)(nrows * ng) * 2u);
+  // (columns past N of an early group read the next group's scales and are not stored)
+  const rsrc_t rs = make_rsrc(a.sp + wn0, nrows > 0 ? ((uint32_t)(ng - 1) * (uint32_t)a.N + (uint32_t)nrows) * 2u : 0u);
   const uint32_t mask = vgpr_const(0x03C003C0u), magic = vgpr_const(0x4C004C00u);
 
   // loop-invariant per-lane offsets; the k offset of a step is a scalar
@@ -2000,7 +2009,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
   for (int y = 0; y < 2; ++y) {
     const int col = 32 * y + l32;
     woff[y] = (uint32_t)(col * (K / 2) + 16 * j);
-    soff[y] = (uint32_t)(col * ng + (G == 32 ? j : 0)) * 2u;
+    soff[y] = ((uint32_t)col + (G == 32 ? (uint32_t)j * (uint32_t)a.N : 0u)) * 2u;
   }
 #pragma unroll
   for (int ss = 0; ss < 4; ++ss) lds_r[ss] = (uint32_t)atile_off(l32, 4 * j + ss) * 2u;
@@ -2035,7 +2044,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
     for (int y = 0; y < 2; ++y) {
       rb[set][y] = __builtin_bit_cast(
           u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rw, (int)(live ? woff[y] : kOob), k0 / 2, 0));
-      rsv[set][y] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(live ? soff[y] : kOob), 2 * (k0 / G), 0);
+      rsv[set][y] = __builtin_amdgcn_raw_buffer_load_b16(rs, (int)(live ? soff[y] : kOob), 2 * (k0 / G) * a.N, 0);
     }
   };
   auto lds_at = [&](uint32_t byte_off) -> u32x4_t* {
@@ -2184,25 +2193,37 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
         }
     __shared__ int s_last;
     if (!splitk_arrive(a.counters + stile, S, &s_last)) return;
+    // (a batch of QB accumulators' loads in flight per piece: each batch and
+    // piece costs the coherent level's whole latency, about 2 us)
+    constexpr int QB = MX == 2 ? 4 : 2;
 #pragma unroll
-    for (int xy = 0; xy < 2 * MX; ++xy) {
-      f32x16_t t = f32x16_t{};
+    for (int q0 = 0; q0 < 2 * MX; q0 += QB) {
+      f32x16_t t[QB];
+#pragma unroll
+      for (int q = 0; q < QB; ++q) t[q] = f32x16_t{};
       for (int z = 0; z < S; ++z) {
         if (z == piece) {
-          t += acc[xy >> 1][xy & 1];
+#pragma unroll
+          for (int q = 0; q < QB; ++q) t[q] += acc[(q0 + q) >> 1][(q0 + q) & 1];
           continue;
         }
-        u32x4_t v[4];
+        u32x4_t v[QB][4];
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          v[c] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
-                                                 rp, (uint32_t)tid * 16u, z * PB + (xy * 4 + c) * NT * 16, 16));
+        for (int q = 0; q < QB; ++q)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
+          for (int c = 0; c < 4; ++c)
+            v[q][c] = __builtin_bit_cast(
+                u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(
+                             rp, (uint32_t)tid * 16u, z * PB + ((q0 + q) * 4 + c) * NT * 16, 16));
 #pragma unroll
-          for (int e = 0; e < 4; ++e) t[4 * c + e] += __uint_as_float(v[c][e]);
+        for (int q = 0; q < QB; ++q)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[q][4 * c + e] += __uint_as_float(v[q][c][e]);
       }
-      acc[xy >> 1][xy & 1] = t;
+#pragma unroll
+      for (int q = 0; q < QB; ++q) acc[(q0 + q) >> 1][(q0 + q) & 1] = t[q];
     }
     splitk_reset(a.counters + stile);
   }
@@ -2227,17 +2248,29 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
   const int K2p = a.K2p;
   const rsrc_t ra2 = make_rsrc(a.a2 + (int64_t)m0 * K2p, (uint32_t)mrows * (uint32_t)K2p * 2u);
   const rsrc_t rb2 = make_rsrc(a.b2 + (int64_t)wn0 * K2p, (uint32_t)nrows * (uint32_t)K2p * 2u);
-  for (int ks = 0; ks < K2p; ks += 16) {
-    u32x4_t bf[2];
+  // (the operands come straight from memory, UB slots of 16 in flight; slots
+  // past K2p read zeros)
+  constexpr int UB = MX == 2 ? 4 : 2;
+  for (int k2 = 0; k2 < K2p; k2 += 16 * UB) {
+    u32x4_t bf[UB][2], af[UB][MX];
 #pragma unroll
-    for (int y = 0; y < 2; ++y)
-      bf[y] = buf_load16(rb2, (uint32_t)((32 * y + l32) * K2p + ks + 8 * j) * 2u);
+    for (int u = 0; u < UB; ++u) {
+      const int ks = k2 + 16 * u + 8 * j;
+      const bool live = k2 + 16 * u < K2p;
 #pragma unroll
-    for (int x = 0; x < MX; ++x) {
-      const u32x4_t af = buf_load16(ra2, (uint32_t)((32 * x + l32) * K2p + ks + 8 * j) * 2u);
-      acc[x][0] = mfma32x32x16<BF16>(af, bf[0], acc[x][0]);
-      acc[x][1] = mfma32x32x16<BF16>(af, bf[1], acc[x][1]);
+      for (int y = 0; y < 2; ++y)
+        bf[u][y] = buf_load16(rb2, live ? (uint32_t)((32 * y + l32) * K2p + ks) * 2u : kOob);
+#pragma unroll
+      for (int x = 0; x < MX; ++x)
+        af[u][x] = buf_load16(ra2, live ? (uint32_t)((32 * x + l32) * K2p + ks) * 2u : kOob);
     }
+#pragma unroll
+    for (int u = 0; u < UB; ++u)
+#pragma unroll
+      for (int x = 0; x < MX; ++x) {
+        acc[x][0] = mfma32x32x16<BF16>(af[u][x], bf[u][0], acc[x][0]);
+        acc[x][1] = mfma32x32x16<BF16>(af[u][x], bf[u][1], acc[x][1]);
+      }
   }
 
   const int gn0 = wn0 + l32;
