@@ -113,8 +113,16 @@ def dtype_code(dtype: torch.dtype) -> int:
         raise ValueError(f"unsupported floating dtype {dtype}") from None
 
 
+def _raw_stream(device: torch.device) -> int:
+    """The handle of the device's current stream, without the torch.cuda.Stream
+    object that current_stream() builds around it on every call."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
+
+
 def stream_handle(device: torch.device):
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+    return ctypes.c_void_p(_raw_stream(device))
 
 
 def call(name: str, *args, device: Optional[torch.device] = None) -> None:
@@ -142,7 +150,7 @@ _WS: dict = {}
 def workspace_buffer(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
     """The uint8 buffer behind workspace() (at least nbytes)."""
     workspace(device, nbytes, kind)
-    return _WS[(device.index, torch.cuda.current_stream(device).cuda_stream, kind)]
+    return _WS[(device.index, _raw_stream(device), kind)]
 
 
 def workspace(device: torch.device, nbytes: int, kind: str):
@@ -152,8 +160,7 @@ def workspace(device: torch.device, nbytes: int, kind: str):
     which must be zero before the first call (every call leaves them zero)."""
     if nbytes <= 0:
         return None, 0
-    stream = torch.cuda.current_stream(device).cuda_stream
-    key = (device.index, stream, kind)
+    key = (device.index, _raw_stream(device), kind)
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)

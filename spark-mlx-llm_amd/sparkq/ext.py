@@ -53,7 +53,7 @@ _REAL = (torch.float16, torch.bfloat16, torch.float32)
 
 
 def _ptr(t):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+    return t.data_ptr() if t is not None else None
 
 
 def _out_buffer(out, shape, dtype, device):
@@ -67,14 +67,15 @@ def _out_buffer(out, shape, dtype, device):
 
 def _require_device(op: str, *tensors):
     for t in tensors:
-        if t is not None and t.device.type != "cuda":
+        if t is not None and not t.is_cuda:
             raise ValueError(f"{op} requires GPU execution")
 
 
 def is_w8a8_available() -> bool:
     """True on a gfx950 device (X/src/spark_w8a8.cpp:204-216 answers the same
     question for Apple M5+)."""
-    if not torch.cuda.is_available():
+    # (an initialized runtime has a device; asking for one costs 1 us a call)
+    if not torch.cuda.is_initialized() and not torch.cuda.is_available():
         return False
     try:
         return bool(_lib.lib().sparkq_is_available())
