@@ -248,10 +248,15 @@ int rms_norm(const void* x, const void* xres, const void* w, float eps, void* hi
 // n = rms_norm(hidden) (spark_mlx_llm/ops/ffn.py:83-105)
 // ---------------------------------------------------------------------------
 // Workspace: the projections' workspace (counters first), then hidden and
-// the normed rows [M][K], act, gate and up [M][I].
+// the normed rows [M][K], act, gate and up [M][I]. The counter block is there
+// for every shape: one that needs no counters leaves them as they are for the
+// next call on the same buffer.
+static size_t ffn_linear_bytes(int64_t M, int64_t K, int64_t I, int G) {
+  return round_up(std::max({w4a16_workspace(M, I, K, G), w4a16_workspace(M, K, I, G), kCounterBytes}),
+                  256);
+}
 size_t ffn_workspace(int64_t M, int64_t K, int64_t I, int G) {
-  const size_t lin = std::max(w4a16_workspace(M, I, K, G), w4a16_workspace(M, K, I, G));
-  return round_up(lin, 256) + 2 * round_up((size_t)(M * K * 2), 256) +
+  return ffn_linear_bytes(M, K, I, G) + 2 * round_up((size_t)(M * K * 2), 256) +
          3 * round_up((size_t)(M * I * 2), 256);
 }
 
@@ -262,9 +267,9 @@ int ffn(const void* x, const void* attn, const void* nw, float eps, const uint32
   const size_t need = ffn_workspace(M, K, I, G);
   if (ws == nullptr || wsb < need)
     return set_error(SPARKQ_ERR_WORKSPACE, "ffn needs a workspace of %zu bytes (got %zu)", need, wsb);
-  const size_t lin = round_up(std::max(w4a16_workspace(M, I, K, G), w4a16_workspace(M, K, I, G)), 256);
+  const size_t lin = ffn_linear_bytes(M, K, I, G);
   unsigned char* p = static_cast<unsigned char*>(ws);
-  void* lws = lin ? p : nullptr;
+  void* lws = p;
   uint16_t* hid = reinterpret_cast<uint16_t*>(p + lin);
   uint16_t* nrm = hid + round_up((size_t)(M * K * 2), 256) / 2;
   uint16_t* act = nrm + round_up((size_t)(M * K * 2), 256) / 2;
@@ -307,10 +312,14 @@ int ffn(const void* x, const void* attn, const void* nw, float eps, const uint32
 // QKV projection of one token + RoPE (X/src/spark_qkv_rope.cpp:83-101)
 // ---------------------------------------------------------------------------
 // Workspace (only when the fused launch does not serve the shape): the
-// projection's workspace, then the [N] projection.
+// projection's workspace with its counter block, for every shape, then the [N]
+// projection.
+static size_t qkv_linear_bytes(int64_t N, int64_t K, int G) {
+  return round_up(std::max(w4a16_workspace(1, N, K, G), kCounterBytes), 256);
+}
 size_t qkv_rope_workspace(int64_t K, int nh, int nkv, int hd, int G) {
   const int64_t N = (int64_t)(nh + 2 * nkv) * hd;
-  return round_up(w4a16_workspace(1, N, K, G), 256) + round_up((size_t)N * 2, 256);
+  return qkv_linear_bytes(N, K, G) + round_up((size_t)N * 2, 256);
 }
 
 int qkv_rope(const void* x, const uint32_t* w, const void* s, const void* b, void* q, void* k,
@@ -324,10 +333,10 @@ int qkv_rope(const void* x, const uint32_t* w, const void* s, const void* b, voi
     return set_error(SPARKQ_ERR_WORKSPACE,
                      "qkv_rope needs a workspace of %zu bytes for this shape (got %zu)", need, wsb);
   const int64_t N = (int64_t)(nh + 2 * nkv) * hd;
-  const size_t lin = round_up(w4a16_workspace(1, N, K, G), 256);
+  const size_t lin = qkv_linear_bytes(N, K, G);
   unsigned char* p = static_cast<unsigned char*>(ws);
   uint16_t* qkv = reinterpret_cast<uint16_t*>(p + lin);
-  if ((rc = w4a16_linear(x, w, s, b, qkv, 1, N, K, G, dt, dt, lin ? p : nullptr, lin, st,
+  if ((rc = w4a16_linear(x, w, s, b, qkv, 1, N, K, G, dt, dt, p, lin, st,
                          nullptr, nullptr)) != 0)
     return rc;
   if ((rc = rope(qkv, q, nh, 1, hd, rd, 0, base, 1.0f, offset, dt, st)) != 0) return rc;

@@ -1071,8 +1071,10 @@ def fused_ffn(x, attention_output, norm_weight, eps: float, gate, up, down, *,
               _lib.stream_handle(dev), device=dev)
     if not return_intermediates:
         return out.view(x.shape)
+    # the projections' workspace, at least the 16 KB counter block
     lin = _round_up(max(_lib.lib().sparkq_w4a16_workspace_bytes(m, inter, k, group_size),
-                        _lib.lib().sparkq_w4a16_workspace_bytes(m, k, inter, group_size)), 256)
+                        _lib.lib().sparkq_w4a16_workspace_bytes(m, k, inter, group_size),
+                        16384), 256)
     hk = _round_up(m * k * 2, 256)
 
     def view(off, n, cols):

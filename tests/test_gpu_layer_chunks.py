@@ -40,6 +40,29 @@ def test_rms_norm_chunks(gpu, k, offset):
             assert d.max() <= 1 and (d == 0).mean() > 0.98
 
 
+def test_ffn_workspace_between_shapes(gpu):
+    """Shapes whose projections need no workspace leave the counters of those
+    that split along k alone: a prompt, a decoded token and the prompt again
+    through one buffer give the prompt's output twice."""
+    import sparkq
+    from test_gpu_layer import _dev, _mat
+
+    k, inter, g = 1024, 2560, 64
+    ws = [_dev(_mat(7, s, n, kk, g, o.BF16), gpu, o.BF16)
+          for s, n, kk in ((4, inter, k), (5, inter, k), (6, k, inter))]
+    nw = up16(o.round16(np.ones(k, np.float32), o.BF16), o.BF16, gpu)
+
+    def run(m):
+        x = up16(o.randn16(m, 1, m * k).reshape(m, k), o.BF16, gpu)
+        return sparkq.fused_ffn(x, x, nw, 1e-6, *ws, group_size=g)
+
+    first = run(70)
+    for m in (1, 2, 5, 16):
+        run(m)
+        print(f"[case] ffn workspace after m={m}", flush=True)
+        assert torch.equal(run(70), first)
+
+
 @pytest.mark.parametrize("m,inter", [(5, 64), (33, 2112), (40, 128)])
 def test_gelu_chunks(gpu, m, inter):
     """act of the composed FFN equals the oracle's gelu(gate) * up of the
@@ -55,7 +78,7 @@ def test_gelu_chunks(gpu, m, inter):
         gate, up = (_mat(m, s, inter, k, g, dtype) for s in (4, 5))
         down = _mat(m, 6, k, inter, g, dtype)
         _, _, nrm, act = (down16(t) for t in sparkq.fused_ffn(
-            up16(x, dtype, gpu), up16(0 * x, dtype, gpu), up16(nw, dtype, gpu), 1e-6,
+            up16(x, dtype, gpu), up16(x[::-1].copy(), dtype, gpu), up16(nw, dtype, gpu), 1e-6,
             _dev(gate, gpu, dtype), _dev(up, gpu, dtype), _dev(down, gpu, dtype), group_size=g,
             return_intermediates=True))
         g16, u16 = (_plain(nrm, t, g, dtype, gpu) for t in (gate, up))
