@@ -1903,6 +1903,8 @@ struct GemmX16Args {
   int gm;  // tile rows per group of the XCD-grouped tile order (0: row-major)
   float* part;
   unsigned* counters;
+  // bf16 [M][N] or null: added to the rounded bf16 output, which rounds again
+  const uint16_t* res;
 };
 
 // Wide variant: a (32*MX) x (64*NWV) tile per workgroup of NWV waves, each
@@ -2274,7 +2276,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
   }
 
   const int gn0 = wn0 + l32;
-  if (a.y_dtype == SPARKQ_BF16 && a.N % 8 == 0 && ((uintptr_t)a.y & 15) == 0) {
+  if (a.y_dtype == SPARKQ_BF16 && a.N % 8 == 0 && (((uintptr_t)a.y | (uintptr_t)a.res) & 15) == 0) {
     // bf16 output through LDS (the A buffers are idle after the main loop's
     // closing barrier): in halves of 64 rows, each wave writes its 64 x 64
     // piece into its own 8 KB of LDS and stores whole 16-byte row segments,
@@ -2295,9 +2297,18 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         const int pc = lane + 64 * i, row = pc >> 3, seg = pc & 7;
-        const u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + row * 128 + seg * 16);
+        u32x4_t v = *reinterpret_cast<const u32x4_t*>(ot + row * 128 + seg * 16);
         const int gm = m0 + 64 * h + row, gn = wn0 + 8 * seg;
-        if (gm < a.M && gn < a.N) *reinterpret_cast<u32x4_t*>(yb + (int64_t)gm * a.N + gn) = v;
+        if (gm < a.M && gn < a.N) {
+          const int64_t idx = (int64_t)gm * a.N + gn;
+          if (a.res) {
+            const u32x4_t r = *reinterpret_cast<const u32x4_t*>(a.res + idx);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              v[e] = pack_round<BF16>(lo16<BF16>(v[e]) + lo16<BF16>(r[e]), hi16<BF16>(v[e]) + hi16<BF16>(r[e]));
+          }
+          *reinterpret_cast<u32x4_t*>(yb + idx) = v;
+        }
       }
     }
     return;
@@ -2313,7 +2324,8 @@ __global__ __launch_bounds__(64 * NWV, 2) void w4_gemm_x16w_kernel(GemmX16Args a
         if (gm < a.M && gn < a.N) {
           const int64_t idx = (int64_t)gm * a.N + gn;
           if (a.y_dtype == SPARKQ_BF16)
-            reinterpret_cast<uint16_t*>(a.y)[idx] = (uint16_t)bf16x2_rne(acc[x][y][v], 0.0f);
+            reinterpret_cast<uint16_t*>(a.y)[idx] =
+                (uint16_t)bf16x2_rne(a.res ? add_rounded<BF16>(acc[x][y][v], a.res[idx]) : acc[x][y][v], 0.0f);
           else
             store_out(a.y, idx, acc[x][y][v], a.y_dtype);
         }
@@ -3024,7 +3036,8 @@ static void launch_gemm_prep(const GemmPrepArgs& p, hipStream_t st) {
 // prep: the weight half made by w4a16_prepare for these scales and biases,
 // or null to compute it in this call's prologue
 static void launch_gemm_x16(int G, const void* x, const uint32_t* w, const void* s,
-                            const void* b, const unsigned char* prep, unsigned* counters,
+                            const void* b, const unsigned char* prep, const void* res,
+                            unsigned* counters,
                             unsigned char* ws, void* y, int ydt, int M, int N, int K,
                             hipStream_t st) {
   const GemmX16Layout l = gemm_x16_layout(M, N, K, G);
@@ -3077,6 +3090,7 @@ static void launch_gemm_x16(int G, const void* x, const uint32_t* w, const void*
   // unchanged); SPARKQ_W4_GEMM_ROWMAJOR keeps the row-major order
   a.gm = env_int("SPARKQ_W4_GEMM_ROWMAJOR", 0) ? 0 : (int)env_int("SPARKQ_W4_GEMM_GM", 4);
   a.part = reinterpret_cast<float*>(ws + l.bytes);
+  a.res = reinterpret_cast<const uint16_t*>(res);
   a.counters = counters;
   dim3 gw((unsigned)wp.items);
 #define SPARKQ_X16W(GG, MM, PP) \
@@ -3138,7 +3152,8 @@ int w4a16_linear(const void* x, const uint32_t* w, const void* s, const void* b,
                  void* ws, size_t wsb, hipStream_t st, const void* res, bool* res_done,
                  const void* prep) {
   // res (16-bit [M][N], y of the same type) is added to the rounded output by
-  // the decode kernels; *res_done says whether the chosen kernel did it
+  // the decode kernels and the bf16 GEMM; *res_done says whether the chosen
+  // kernel did it
   if (res_done) *res_done = false;
   const size_t need = w4a16_workspace(M, N, K, G);
   if (need > 0 && (ws == nullptr || wsb < need))
@@ -3261,8 +3276,10 @@ int w4a16_linear(const void* x, const uint32_t* w, const void* s, const void* b,
   }
   unsigned char* wsp = reinterpret_cast<unsigned char*>(ws) + kCounterBytes;
   if (xdt == SPARKQ_BF16) {
+    const bool add = res != nullptr && ydt == SPARKQ_BF16;
+    if (res_done) *res_done = add;
     launch_gemm_x16(G, x, w, s, b, reinterpret_cast<const unsigned char*>(prep),
-                    reinterpret_cast<unsigned*>(ws), wsp, y, ydt, (int)M, (int)N,
+                    add ? res : nullptr, reinterpret_cast<unsigned*>(ws), wsp, y, ydt, (int)M, (int)N,
                     (int)K, st);
     return check_launch("w4_gemm_x16w_kernel");
   }

@@ -63,10 +63,12 @@ def test_ffn_workspace_between_shapes(gpu):
         assert torch.equal(run(70), first)
 
 
-@pytest.mark.parametrize("m,inter", [(5, 64), (33, 2112), (40, 128)])
+@pytest.mark.parametrize("m,inter", [(5, 64), (33, 2112), (40, 128), (129, 320)])
 def test_gelu_chunks(gpu, m, inter):
     """act of the composed FFN equals the oracle's gelu(gate) * up of the
-    device's own projections, bit for bit."""
+    device's own projections, and its output the down projection rounded, plus
+    the residual, rounded again (in the bf16 GEMM's epilogue, over whole and
+    split tiles), bit for bit."""
     import sparkq
     from test_gpu_layer import _dev, _mat, _plain
 
@@ -77,9 +79,10 @@ def test_gelu_chunks(gpu, m, inter):
         nw = o.round16(np.ones(k, np.float32), dtype)
         gate, up = (_mat(m, s, inter, k, g, dtype) for s in (4, 5))
         down = _mat(m, 6, k, inter, g, dtype)
-        _, _, nrm, act = (down16(t) for t in sparkq.fused_ffn(
+        out, hid, nrm, act = (down16(t) for t in sparkq.fused_ffn(
             up16(x, dtype, gpu), up16(x[::-1].copy(), dtype, gpu), up16(nw, dtype, gpu), 1e-6,
             _dev(gate, gpu, dtype), _dev(up, gpu, dtype), _dev(down, gpu, dtype), group_size=g,
             return_intermediates=True))
         g16, u16 = (_plain(nrm, t, g, dtype, gpu) for t in (gate, up))
         assert np.array_equal(act, o.gelu_mul16(g16, u16, dtype))
+        assert np.array_equal(out, o.add16(hid, _plain(act, down, g, dtype, gpu), dtype))
