@@ -1174,12 +1174,23 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void sdpa_prefill_affine_ker
       float mm = kNegInf;
       for (int c = 0; c < S; ++c) mm = fmaxf(mm, splitk_load(a.pm + (pbase + c) * 128 + rrow));
       float z = 0.0f;
+      f32x4_t own[NJ];
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) acc[rt][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < NJ; ++j) {
+        own[j] = acc[rt][j];
+        acc[rt][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+      }
       for (int c = 0; c < S; ++c) {
         const float mc = splitk_load(a.pm + (pbase + c) * 128 + rrow);
         const float w = exp2_guarded(mc - mm, mc != kNegInf);
         z = fmaf(splitk_load(a.pz + (pbase + c) * 128 + rrow), w, z);
+        if (c == chunk) {  // this workgroup's own chunk, from its registers
+#pragma unroll
+          for (int j = 0; j < NJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[rt][j][r] = fmaf(own[j][r], w, acc[rt][j][r]);
+          continue;
+        }
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
@@ -1766,9 +1777,15 @@ static void launch_prefill_affine_d(const SdpaArgs& a, int qdt, dim3 grid, hipSt
 // paired grid still has a workgroup for every CU (D <= 128); a grid short of
 // one workgroup per CU splits each tile's blocks over S <= 8 workgroups,
 // merged in the same launch through the workspace (tile counters, then the
-// per-chunk maxima, sums and accumulators).
+// per-chunk maxima, sums and accumulators). At head dim 256, where a workgroup
+// has a CU to itself, one round of causal tiles lasts as long as its longest
+// one: from one to two tiles per CU each is split in two, whose halves, longest
+// first, even out (16/4 heads, L = N = 2048: 142 us -> 115), as long as the
+// context is at most half as long again as the queries (N is known at the
+// launch only); with longer ones the tiles are nearly alike.
 struct AffPrefillPlan {
   int pair, S;
+  bool halves;
   int64_t ntiles_all;
   size_t bytes;
 };
@@ -1785,6 +1802,9 @@ static AffPrefillPlan plan_prefill_affine(int64_t B, int64_t Hq, int64_t Hkv, in
   }();
   if (!p.pair && p.ntiles_all < target && p.ntiles_all <= (int64_t)(kCounterBytes / 4))
     p.S = (int)std::min<int64_t>(8, cdiv(target, p.ntiles_all));
+  else if (D == 256 && causal && p.ntiles_all >= 256 && p.ntiles_all < 512 &&
+           !env_int("SPARKQ_PREFILL_NO_HALVES", 0))
+    p.S = 2, p.halves = true;
   p.bytes = p.S > 1 ? kCounterBytes + round_up((size_t)p.ntiles_all * p.S * 128 * 4, 256) * 2 +
                           (size_t)p.ntiles_all * p.S * 128 * D * 4
                     : 0;
@@ -1801,7 +1821,8 @@ int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, co
                                int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
                                int64_t D, int G, int causal, int qdt, int odt, float scale,
                                const int64_t* strides, void* ws, size_t wsb, hipStream_t st) {
-  const AffPrefillPlan plan = plan_prefill_affine(B, Hq, Hkv, L, D, causal);
+  AffPrefillPlan plan = plan_prefill_affine(B, Hq, Hkv, L, D, causal);
+  if (plan.halves && 2 * N > 3 * L) plan.S = 1;
   if (plan.S > 1 && (ws == nullptr || wsb < plan.bytes))
     return set_error(SPARKQ_ERR_WORKSPACE, "int8kv_sdpa_prefill_affine: workspace too small");
   SdpaArgs a{};

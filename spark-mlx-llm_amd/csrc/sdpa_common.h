@@ -38,16 +38,20 @@ struct SdpaArgs {
 // takes a contiguous chunk of the (y, x) order: the row tiles of one
 // (sequence, KV head) share an XCD's L2 for their K/V blocks, and within a
 // chunk the items keep their relative order (the longest causal tiles still
-// start first). A bijection on the grid; a grid of a size not divisible by
-// 8 keeps its order.
+// start first). Where k XCDs share one (sequence, KV head), each takes every
+// k-th of its items: contiguous runs would leave the long causal tiles to one
+// XCD and the short ones to another. A bijection on the grid; a grid of a size
+// not divisible by 8 keeps its order.
 __device__ __forceinline__ void xcd_grid_item(bool xcd, int& x, int& y) {
   x = (int)blockIdx.x;
   y = (int)blockIdx.y;
   const int gx = (int)gridDim.x, T = gx * (int)gridDim.y;
   if (!xcd || (T & 7) != 0) return;
-  const int id = y * gx + x, v = (id & 7) * (T >> 3) + (id >> 3);
+  const int id = y * gx + x, m = T >> 3, v = (id & 7) * m + (id >> 3);
   y = v / gx;
   x = v - y * gx;
+  const int k = gx / m;
+  if (k > 1 && k * m == gx) x = x % m * k + x / m;
 }
 
 constexpr float kNegInf = -__builtin_huge_valf();
