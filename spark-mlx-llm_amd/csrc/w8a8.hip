@@ -34,6 +34,8 @@
 //                        workgroup slot (gate+up): one round of workgroups
 //                        owning up to three tiles each, the activation tile
 //                        staged once per workgroup in LDS.
+#include <type_traits>
+
 #include "common.h"
 
 namespace sparkq {
@@ -1268,13 +1270,14 @@ static bool use_rows_sync(int64_t M, int64_t K, int xdt) {
 // Tiled int8 GEMM for prefill sizes (i8_gemm_kernel)
 // ---------------------------------------------------------------------------
 // The reference serves out_proj at any M with a BM128 x BN128 x BK512
-// tensor-op GEMM (X/src/spark_w8a8.cpp:120-150). Here: a 128 x 128 tile per
-// workgroup of four waves in a 2 x 2 arrangement, each wave 64 x 64 (two
-// 32-row by two 32-column fragments of v_mfma_i32_32x32x32_i8). A k step is
+// tensor-op GEMM (X/src/spark_w8a8.cpp:120-150). Here: a 64*FR x 64*FR tile
+// (FR = 1 or 2) per workgroup of four waves in a 2 x 2 arrangement, each wave
+// FR x FR fragments of v_mfma_i32_32x32x32_i8. A k step is
 // 128 bytes of every row of both operands, staged through LDS (double
 // buffered; 128-byte rows whose 16-byte chunks are swizzled by the row, so
 // the 32 rows a fragment read touches at one chunk index fall on distinct
-// banks); the loads of step s+1 go out before the MFMAs of step s. Lane
+// banks); the loads of step s+2 go out before the MFMAs of step s (at 128-row
+// tiles within 2% of one step ahead; small grids wait for their loads). Lane
 // (l % 32, l / 32) of a fragment holds bytes 16 * (l / 32) .. +15 of row
 // l % 32 of a 32-k sub-step, for activations and weights alike. Grids with
 // fewer tiles than CUs split K into S pieces: each piece stores
@@ -1295,8 +1298,9 @@ __device__ __forceinline__ uint32_t i8_tile_off(int row, int kc) {
   return (uint32_t)(row * 128 + ((kc ^ ((t ^ (t >> 3)) & 7)) << 4));
 }
 
+template <int FR>
 __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
-  constexpr int BM = 128, BN = 128, TB = (BM + BN) * kI8GK;  // bytes per stage
+  constexpr int BM = 64 * FR, BN = BM, TB = (BM + BN) * kI8GK;  // bytes per stage
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * TB];
   __shared__ int s_last;
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1333,7 +1337,7 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
   const rsrc_t rb = make_rsrc(a.b + (int64_t)n0 * K, (uint32_t)nr * (uint32_t)K);
 
   // staging: chunk p = tid + 256 i of each operand, row p / 8, chunk p % 8
-  constexpr int CH = BM * 8 / 256;  // chunks per thread and operand (4)
+  constexpr int CH = BM * 8 / 256;  // chunks per thread and operand
   uint32_t goff[CH], loff[CH];
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
@@ -1341,70 +1345,84 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
     goff[i] = (uint32_t)(row * K + kc * 16);
     loff[i] = i8_tile_off(row, kc);
   }
-  u32x4_t va[CH], vb[CH];
-  auto load = [&](int step) {
-    const int k0 = step * kI8GK;
+  // register set t holds the loads of the steps of parity t; past the last
+  // step they go to an out-of-range offset (zeros), so that no branch splits
+  // the wait counts
+  u32x4_t va[2][CH], vb[2][CH];
+  auto load = [&](int step, int set) {
+    const bool live = step < s_end;
+    const int k0 = live ? step * kI8GK : 0;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-      va[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, (int)goff[i], k0, 0));
-      vb[i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, (int)goff[i], k0, 0));
+      const int o = (int)(live ? goff[i] : kOob);
+      va[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(ra, o, k0, 0));
+      vb[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, o, k0, 0));
     }
   };
   auto stage = [&](int buf) {
     unsigned char* base = lds + buf * TB;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-      *reinterpret_cast<u32x4_t*>(base + loff[i]) = va[i];
-      *reinterpret_cast<u32x4_t*>(base + BM * kI8GK + loff[i]) = vb[i];
+      *reinterpret_cast<u32x4_t*>(base + loff[i]) = va[buf][i];
+      *reinterpret_cast<u32x4_t*>(base + BM * kI8GK + loff[i]) = vb[buf][i];
     }
   };
 
-  i32x16_t acc[2][2];
+  i32x16_t acc[FR][FR];
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int x = 0; x < FR; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) acc[x][y] = i32x16_t{};
+    for (int y = 0; y < FR; ++y) acc[x][y] = i32x16_t{};
   // fragment rows (a multiple of 32 plus l32: the swizzle's t is l32)
-  const int ar0 = wm * 64 + l32, br0 = wn * 64 + l32;
+  const int ar0 = wm * 32 * FR + l32, br0 = wn * 32 * FR + l32;
 
-  if (s_begin < s_end) {
-    load(s_begin);
-    stage(0);
-    __syncthreads();
-  }
-  for (int step = s_begin; step < s_end; ++step) {
-    const int cur = (step - s_begin) & 1;
-    const bool more = step + 1 < s_end;
-    if (more) load(step + 1);
+  auto body = [&](int step, auto curc) {
+    constexpr int cur = decltype(curc)::value;
+    __builtin_amdgcn_sched_barrier(0);
+    load(step + 2, cur);
     const unsigned char* base = lds + cur * TB;
 #pragma unroll
     for (int ss = 0; ss < 4; ++ss) {
       const int kc = 2 * ss + j;
-      u32x4_t af[2], bf[2];
+      u32x4_t af[FR], bf[FR];
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int x = 0; x < FR; ++x)
         af[x] = *reinterpret_cast<const u32x4_t*>(base + i8_tile_off(ar0 + 32 * x, kc));
 #pragma unroll
-      for (int y = 0; y < 2; ++y)
+      for (int y = 0; y < FR; ++y)
         bf[y] = *reinterpret_cast<const u32x4_t*>(base + BM * kI8GK + i8_tile_off(br0 + 32 * y, kc));
 #pragma unroll
-      for (int x = 0; x < 2; ++x)
+      for (int x = 0; x < FR; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y) acc[x][y] = mfma_i8(af[x], bf[y], acc[x][y]);
+        for (int y = 0; y < FR; ++y) acc[x][y] = mfma_i8(af[x], bf[y], acc[x][y]);
     }
-    if (more) stage(cur ^ 1);
+    stage(cur ^ 1);  // (last read in the step before, behind its barrier)
+    __syncthreads();
+  };
+  if (s_begin < s_end) {
+    load(s_begin, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    load(s_begin + 1, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    stage(0);
     __syncthreads();
   }
+  int step = s_begin;
+  for (; step + 2 <= s_end; step += 2) {
+    body(step, std::integral_constant<int, 0>{});
+    body(step + 1, std::integral_constant<int, 1>{});
+  }
+  if (step < s_end) body(step, std::integral_constant<int, 0>{});
 
   if (S > 1) {
     // this piece's tile: chunk c (16 bytes) of every thread at (c * 256 + tid) * 16
-    constexpr uint32_t PB = 4 * 16 * 4 * 256;  // bytes per piece
+    constexpr uint32_t PB = FR * FR * 16 * 4 * 256;  // bytes per piece
     const rsrc_t rp = make_rsrc(a.part + (size_t)si * S * (PB / 4), (uint32_t)S * PB);
 #pragma unroll
-    for (int xy = 0; xy < 4; ++xy)
+    for (int xy = 0; xy < FR * FR; ++xy)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const i32x16_t& v = acc[xy >> 1][xy & 1];
+        const i32x16_t& v = acc[xy / FR][xy % FR];
         const u32x4_t w = {(uint32_t)v[4 * q], (uint32_t)v[4 * q + 1], (uint32_t)v[4 * q + 2],
                            (uint32_t)v[4 * q + 3]};
         __builtin_amdgcn_raw_buffer_store_b128(w, rp, (uint32_t)tid * 16u,
@@ -1412,8 +1430,8 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
       }
     if (!splitk_arrive(a.counters + si, S, &s_last)) return;
 #pragma unroll
-    for (int xy = 0; xy < 4; ++xy) {
-      i32x16_t t = acc[xy >> 1][xy & 1];
+    for (int xy = 0; xy < FR * FR; ++xy) {
+      i32x16_t t = acc[xy / FR][xy % FR];
       for (int z = 0; z < S; ++z) {
         if (z == piece) continue;
 #pragma unroll
@@ -1424,19 +1442,19 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
           for (int e = 0; e < 4; ++e) t[4 * q + e] += (int32_t)w[e];
         }
       }
-      acc[xy >> 1][xy & 1] = t;
+      acc[xy / FR][xy % FR] = t;
     }
     splitk_reset(a.counters + si);
   }
 
 #pragma unroll
-  for (int x = 0; x < 2; ++x)
+  for (int x = 0; x < FR; ++x)
 #pragma unroll
-    for (int y = 0; y < 2; ++y) {
-      const int gn = n0 + wn * 64 + 32 * y + l32;
+    for (int y = 0; y < FR; ++y) {
+      const int gn = n0 + wn * 32 * FR + 32 * y + l32;
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int gm = m0 + wm * 64 + 32 * x + mfma32_row(lane, v);
+        const int gm = m0 + wm * 32 * FR + 32 * x + mfma32_row(lane, v);
         if (gm < M && gn < N) i8_store(a, gm, gn, acc[x][y][v]);
       }
     }
@@ -1707,7 +1725,7 @@ static I8Plan plan_i8(int64_t M, int64_t N, int64_t K) {
 // least eight steps (tiles within the counter block).
 struct I8GemmPlan {
   bool ok;
-  int tiles_n, tiles, S, full;
+  int FR, tiles_n, tiles, S, full;
   size_t part_bytes;
 };
 
@@ -1715,7 +1733,13 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
   I8GemmPlan p{};
   if (M < env_int("SPARKQ_I8_GEMM_FROM", 64) || env_int("SPARKQ_I8_NO_GEMM", 0)) return p;
   if (K % kI8GK != 0 || (int64_t)kI8GK * K >= (int64_t)kOob) return p;
-  const int64_t tn = cdiv(N, 128), tiles = cdiv(M, 128) * tn, cus = device_cus();
+  const int64_t cus = device_cus();
+  // 64-row tiles where 128-row ones would not give every CU one: 512 x 2560 x
+  // 4096 42.0 -> 26.2 us a call, 64 x 2560 x 4096 32.9 -> 16.4, 200 x 2560 x
+  // 9728 42.8 -> 28.6; from one per CU the larger tiles' fewer LDS reads win
+  // (2048 x 2560 x 4096, 320 of them: 58.6 against 52.8 us)
+  p.FR = cdiv(M, 128) * cdiv(N, 128) < env_int("SPARKQ_I8_GEMM_SMALL", cus) ? 1 : 2;
+  const int64_t B = 64 * p.FR, tn = cdiv(N, B), tiles = cdiv(M, B) * tn;
   if (tiles * 4 > (int64_t)0x7FFFFFFF) return p;
   // Fewer tiles than CUs: every tile split in S pieces. Between one and two
   // tiles per CU (M=2048 out_proj: 320 tiles on 256 CUs), one whole tile per
@@ -1734,6 +1758,9 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
       full = cus;
     }
   }
+  // long rows on more small tiles than run at once: halves even out the last
+  // round (1000 x 2560 x 9728, 640 tiles: 65.7 -> 62.3 us)
+  if (p.FR == 1 && S == 1 && tiles > 2 * cus && K / kI8GK >= 64 && tiles <= kMaxCounterTiles) S = 2;
   if (env_int("SPARKQ_I8_GEMM_SPLITS", 0) > 0 && tiles <= kMaxCounterTiles) {
     S = std::min<int64_t>(env_int("SPARKQ_I8_GEMM_SPLITS", 1), K / kI8GK);
     full = 0;
@@ -1742,7 +1769,7 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
   p.tiles = (int)tiles;
   p.S = (int)std::max<int64_t>(S, 1);
   p.full = p.S > 1 ? (int)full : (int)tiles;
-  p.part_bytes = p.S > 1 ? round_up((size_t)(tiles - p.full) * p.S * 65536, 256) : 0;
+  p.part_bytes = p.S > 1 ? round_up((size_t)(tiles - p.full) * p.S * B * B * 4, 256) : 0;
   p.ok = true;
   return p;
 }
@@ -1774,8 +1801,11 @@ static int launch_i8_gemm(I8Args args, const I8GemmPlan& p, hipStream_t st) {
   args.tiles = p.tiles;
   args.S = p.S;
   args.full = p.full;
-  hipLaunchKernelGGL(i8_gemm_kernel, dim3((unsigned)(p.full + (p.tiles - p.full) * p.S)), dim3(256), 0, st,
-                     args);
+  const dim3 grid((unsigned)(p.full + (p.tiles - p.full) * p.S));
+  if (p.FR == 1)
+    hipLaunchKernelGGL(i8_gemm_kernel<1>, grid, dim3(256), 0, st, args);
+  else
+    hipLaunchKernelGGL(i8_gemm_kernel<2>, grid, dim3(256), 0, st, args);
   return check_launch("i8_gemm_kernel");
 }
 

@@ -1,0 +1,23 @@
+"""The tiled int8 GEMM in both tile sizes at the edges of its tiles, steps and
+pieces: int32 sums equal torch's on the CPU exactly, whatever the split."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("small", ["1", "100000"])  # 128- and 64-row tiles
+@pytest.mark.parametrize("m,n,k,pieces", [(64, 1, 128, 1), (65, 63, 384, 1), (127, 65, 1152, 3),
+                                          (129, 130, 256, 2), (200, 257, 1280, 4), (320, 192, 640, 0)])
+def test_i8_tiles_exact(gpu, small, m, n, k, pieces, monkeypatch):
+    import sparkq
+
+    print(f"[case] i8 tiles small={small} m={m} n={n} k={k} pieces={pieces}", flush=True)
+    monkeypatch.setenv("SPARKQ_I8_GEMM_SMALL", small)
+    if pieces:
+        monkeypatch.setenv("SPARKQ_I8_GEMM_SPLITS", str(pieces))
+    gen = torch.Generator().manual_seed(m + n + k)
+    a, b = (torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int8) for r in (m, n))
+    y = sparkq.int8_matmul_int32(a.to(gpu), b.to(gpu)).cpu()
+    assert torch.equal(y, a.to(torch.int32) @ b.to(torch.int32).T)
