@@ -1746,11 +1746,13 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
   // CU and the tiles past them split in S pieces, so that every CU runs one
   // whole tile and at most one piece instead of a quarter of the CUs running
   // two whole tiles (the whole call at M=2048, N=2560, K=4096: 64.0-64.1 ->
-  // 57.7-59.3 us; SPARKQ_I8_GEMM_NO_CU1 keeps the unsplit grid).
+  // 57.7-59.3 us; SPARKQ_I8_GEMM_NO_CU1 keeps the unsplit grid). Exactly one
+  // tile per CU is a whole round already and stays unsplit (512 x 2048 x 4096
+  // 23.3 us, in 128-row tiles and four pieces 38.0).
   int64_t S = 1, full = 0;
   if (tiles < cus && tiles <= kMaxCounterTiles) {
     S = std::min<int64_t>(std::min<int64_t>(4, 2 * cus / tiles), std::max<int64_t>(1, (K / kI8GK) / 8));
-  } else if (tiles < 2 * cus && !env_int("SPARKQ_I8_GEMM_NO_CU1", 0)) {
+  } else if (tiles > cus && tiles < 2 * cus && !env_int("SPARKQ_I8_GEMM_NO_CU1", 0)) {
     const int64_t rest = tiles - cus;
     const int64_t s = std::min<int64_t>(std::min<int64_t>(4, cus / rest), std::max<int64_t>(1, (K / kI8GK) / 8));
     if (s > 1 && rest <= kMaxCounterTiles) {
@@ -1759,7 +1761,9 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
     }
   }
   // long rows on more small tiles than run at once: halves even out the last
-  // round (1000 x 2560 x 9728, 640 tiles: 65.7 -> 62.3 us)
+  // round (1000 x 2560 x 9728, 640 tiles: 63.8 -> 60.9 us; 1000 x 2560 x 8192
+  // 56.7 -> 53.9, 800 x 4096 x 8192, 832 tiles, 68.6 -> 66.3; shorter rows gain
+  // nothing: K = 6144 44.4 -> 43.6, K = 4096 33.4 -> 35.0)
   if (p.FR == 1 && S == 1 && tiles > 2 * cus && K / kI8GK >= 64 && tiles <= kMaxCounterTiles) S = 2;
   if (env_int("SPARKQ_I8_GEMM_SPLITS", 0) > 0 && tiles <= kMaxCounterTiles) {
     S = std::min<int64_t>(env_int("SPARKQ_I8_GEMM_SPLITS", 1), K / kI8GK);

@@ -21,3 +21,19 @@ def test_i8_tiles_exact(gpu, small, m, n, k, pieces, monkeypatch):
     a, b = (torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int8) for r in (m, n))
     y = sparkq.int8_matmul_int32(a.to(gpu), b.to(gpu)).cpu()
     assert torch.equal(y, a.to(torch.int32) @ b.to(torch.int32).T)
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1020, 960, 2048), (512, 2048, 4096), (1000, 1020, 1024), (64, 16448, 2048),  # 240, 256, 256, 257 tiles
+    (448, 4672, 2048), (512, 4096, 2048), (1216, 1728, 2048), (640, 4000, 8192),  # 511, 512, 513, 630
+    (2048, 2048, 2048), (2048, 2176, 2048), (4096, 2048, 2048),  # 256, 272 and 512 tiles of 128 rows
+])
+def test_i8_planned_exact(gpu, m, n, k):
+    """The planner's own tiles and pieces around one and two tiles per CU."""
+    import sparkq
+
+    print(f"[case] i8 plan m={m} n={n} k={k}", flush=True)
+    gen = torch.Generator().manual_seed(m + n + k)
+    a, b = (torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int8) for r in (m, n))
+    y = sparkq.int8_matmul_int32(a.to(gpu), b.to(gpu)).cpu()
+    assert torch.equal(y.double(), a.double() @ b.double().T)
