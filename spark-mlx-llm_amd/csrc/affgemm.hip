@@ -1,11 +1,18 @@
 // affgemm.hip -- matmul over groupwise affine weights whose scales do not fit
 // into a 16-bit operand: 4-bit weights of float16 checkpoints (from 33 rows)
-// and 8-bit weights with scales of any dtype (any number of rows),
-//   y[m,n] = sum_g s[n,g] * (sum_{k in g} x[m,k] q[n,k]) + b[n,g] * X[m,g],
-// X[m,g] the sum of x over group g. Nothing is rounded below fp32: codes 0..15
-// and 0..255 are exact 16-bit operands, the products of a group accumulate in
-// fp32 on the 32x32x16 MFMA, each group's sum enters y with one fp32 FMA by
-// its scale, and the bias part is an fp32 MFMA (32x32x2) over the groups.
+// and 8-bit weights with scales of any dtype (any number of rows). With the
+// codes centred, c = q - 2^(bits-1) and b' = b + 2^(bits-1) s,
+//   y[m,n] = sum_g s[n,g] * (sum_{k in g} x[m,k] c[n,k]) + b'[n,g] * X[m,g],
+// X[m,g] the sum of x over group g. Nothing is rounded below fp32: centred
+// codes are exact 16-bit operands, the products of a group accumulate in fp32
+// on the 32x32x16 MFMA, each group's sum enters y with one fp32 FMA by its
+// scale, and its bias part follows at once on the fp32 MFMA (32x32x1, two
+// blocks). A running sum of the scale parts alone would reach hundreds of
+// times the result before the bias parts cancel it. Relative error of the fp32
+// output against float64, activations of mean 0 / mean 1: fp16 4-bit
+// 512 x 3584 x 2560 G64 1.6e-7 / 1.7e-7, 333 x 2560 x 9728 G32 2.3e-7 / 2.3e-7,
+// bf16 8-bit 512 x 3584 x 2560 G64 1.6e-7 / 1.7e-7 (uncentred codes, group by
+// group 1.8e-7 / 5.9e-7; uncentred with all bias parts last 4.3e-7 / 1.0e-5).
 //
 // affine_prep_kernel turns scales and biases into fp32 [K/G][N] (a wave's 32
 // columns in one 128-byte line; in [N][K/G] order each of them costs a line of
@@ -17,18 +24,20 @@
 // bytes. Activations go through LDS (rows of 16 chunks of 16 bytes, chunk c of
 // row r at c ^ (r & 15): operand reads of 16 rows touch every bank once), each
 // wave loads its own codes into registers and decodes them there; the loads of
-// unit u+2 go out in unit u. Where the tiles do not fill the chip, pieces of K
-// go to workgroups of their own and affine_sum_kernel adds their fp32 sums in
-// order.
+// unit u+2 go out in unit u. The compiler places them late in the unit, and
+// the scales (of bf16 8-bit weights some codes too) move to other registers at
+// the end of every second unit, which waits for loads just issued. Where the
+// tiles do not fill the chip, pieces of K go to workgroups of their own and
+// affine_sum_kernel adds their fp32 sums in order.
 //
-// What bounds it: at few tiles the latency of the units' chain; where two
-// workgroups share a CU, LDS reads (0.27 us per unit), the VALU (0.25) and the
-// MFMA (0.21) take turns, 0.75 us in all. 64 columns per wave, which would
-// halve the LDS reads, have no registers for it and measured 0-20% slower.
-// Per call, against the kernels this replaced: fp16 4-bit 333 x 2560 x 9728
-// G128 235 -> 46 us, 512 x 3584 x 2560 G64 69 -> 42, 2048 x 19456 x 2560 G64
-// 361 -> 311 (658 TFLOP/s); bf16 8-bit 512 x 3584 x 2560 G64 102 -> 42,
-// 700 x 19456 x 2560 G32 1245 -> 201.
+// What bounds it: the latency of the units' chain, at many tiles the turns that
+// LDS reads, the VALU and the MFMA take (about 0.25 us a unit each). 64
+// columns per wave, which would halve the LDS reads, have no registers for it
+// and measured 0-20% slower. 4-bit instances fit three workgroups on a CU, 8-bit
+// ones two. Per call, against the kernels this replaced: fp16 4-bit 333 x 2560 x
+// 9728 G128 234 -> 45 us, 512 x 3584 x 2560 G64 68 -> 34, 2048 x 19456 x 2560
+// G64 371 -> 314 (650 TFLOP/s); bf16 8-bit 512 x 3584 x 2560 G64 104 -> 39,
+// 700 x 19456 x 2560 G32 1258 -> 180.
 #include <algorithm>
 #include <type_traits>
 
@@ -42,10 +51,12 @@ struct AffPrepArgs {
   const uint16_t* x;   // [M][K]
   const void* sc;      // [N][ng] in the scale dtype
   const void* bi;
-  float* st;           // [ng][N]
-  float* bt;           // [ng][N]
-  float* xs;           // [ng][M]
+  float* st;           // [ngp][N]
+  float* bt;           // [ngp][N]: b + centre * s
+  float* xs;           // [ngp][M]
   int M, N, K, G, s_dtype;
+  int ngp;             // groups of whole units; those past K are zeros
+  float centre;        // of the codes: 8 or 128
   int wblocks;         // blocks of the weight half (dispatched first)
 };
 
@@ -57,21 +68,22 @@ __global__ __launch_bounds__(256) void affine_prep_kernel(AffPrepArgs a) {
   __shared__ float ts[32][65], tb[32][65];
   const int tid = threadIdx.x, ng = a.K / a.G;
   if ((int)blockIdx.x < a.wblocks) {
-    const int gb = (ng + 31) / 32;
+    const int gb = (a.ngp + 31) / 32;
     const int n0 = (int)blockIdx.x / gb * 64, g0 = (int)blockIdx.x % gb * 32;
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int n = n0 + (tid >> 5) + 8 * i, g = g0 + (tid & 31);
       const bool live = n < a.N && g < ng;
       const int64_t at = live ? (int64_t)n * ng + g : 0;
-      ts[tid & 31][(tid >> 5) + 8 * i] = load_in(a.sc, at, a.s_dtype);
-      tb[tid & 31][(tid >> 5) + 8 * i] = load_in(a.bi, at, a.s_dtype);
+      const float sc = load_in(a.sc, at, a.s_dtype), bi = load_in(a.bi, at, a.s_dtype);
+      ts[tid & 31][(tid >> 5) + 8 * i] = live ? sc : 0.0f;
+      tb[tid & 31][(tid >> 5) + 8 * i] = live ? fmaf(a.centre, sc, bi) : 0.0f;
     }
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       const int gl = (tid >> 6) + 4 * i, n = n0 + (tid & 63), g = g0 + gl;
-      if (n < a.N && g < ng) {
+      if (n < a.N && g < a.ngp) {
         a.st[(int64_t)g * a.N + n] = ts[gl][tid & 63];
         a.bt[(int64_t)g * a.N + n] = tb[gl][tid & 63];
       }
@@ -91,44 +103,49 @@ __global__ __launch_bounds__(256) void affine_prep_kernel(AffPrepArgs a) {
   for (int o = 1; o < cpg; o <<= 1) s += __shfl_xor(s, o);
   const int m = (int)(c / nc), cc = (int)(c - (int64_t)m * nc);
   if ((cc & (cpg - 1)) == 0) a.xs[(int64_t)(cc / cpg) * a.M + m] = s;
+  if (cc == nc - 1)
+    for (int g = ng; g < a.ngp; ++g) a.xs[(int64_t)g * a.M + m] = 0.0f;
 }
 
 struct AffGemmArgs {
   const uint16_t* x;   // [M][K]
   const uint32_t* w;   // [N][K*BITS/32]
-  const float* st;     // [ng][N]
-  const float* bt;     // [ng][N]
-  const float* xs;     // [ng][M]
+  const float* st;     // [ngp][N]
+  const float* bt;     // [ngp][N], b + centre * s
+  const float* xs;     // [ngp][M]
   void* y;             // [M][N]
   float* part;         // [S][M][N] when S > 1
   int y_dtype, M, N, K, tiles_m, tiles_n, S;
 };
 
+typedef float f32x32_t __attribute__((ext_vector_type(32)));
+
 constexpr int kAffBM = 64, kAffBN = 128, kAffBK = 128;
 
-// a chunk's 8 codes as exact 16-bit values in k order
+// a chunk's 8 codes minus 2^(BITS-1) as exact 16-bit values in k order
 template <typename T, int BITS>
 __device__ __forceinline__ u32x4_t aff_decode(const uint32_t* w, DecodeConsts dc) {
   u32x4_t r;
   if constexpr (BITS == 4) {
     static_assert(T::kExactDecode, "4-bit codes are decoded exactly for fp16 only");
-    r = decode_w4<T>(w[0], dc);
+    r = decode_w4<T, 8>(w[0], dc);
   } else if constexpr (T::code == SPARKQ_F16) {
 #pragma unroll
     for (int i = 0; i < 4; ++i)  // bytes under fp16 1024, which an exact subtract removes
-      r[i] = exact_f16_pair(
+      r[i] = exact_f16_pair<128>(
           __builtin_amdgcn_perm(0x64646464u, w[i >> 1], (i & 1) ? 0x04030402u : 0x04010400u));
   } else {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      r[i] = pack_round<T>((float)((w[i >> 1] >> (16 * (i & 1))) & 255u),
-                           (float)((w[i >> 1] >> (16 * (i & 1) + 8)) & 255u));
+    for (int i = 0; i < 4; ++i) {  // c ^ 128 as a signed byte is c - 128
+      const int v = (int)(w[i >> 1] ^ 0x80808080u) >> (16 * (i & 1));
+      r[i] = pack_round<T>((float)(signed char)v, (float)(signed char)(v >> 8));
+    }
   }
   return r;
 }
 
 template <typename T, int BITS, int G>
-__global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
+__global__ __launch_bounds__(256, BITS == 4 ? 3 : 2) void affine_gemm_kernel(AffGemmArgs a) {
   constexpr int WC = BITS / 4;          // words per chunk of 8 codes
   constexpr int WQ = 2 * WC;            // 16-byte code loads per unit and column
   constexpr int NGU = kAffBK / G;       // groups per unit
@@ -138,7 +155,7 @@ __global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane >> 5, l32 = lane & 31;
-  const int K = a.K, N = a.N, M = a.M, ng = K / G;
+  const int K = a.K, N = a.N, M = a.M;
   // XCD-contiguous chunks of the (piece, tile) order, the tiles of a piece in
   // groups of 8 tile rows column by column: what an XCD runs together shares
   // activation rows and weight columns in its L2
@@ -175,7 +192,7 @@ __global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
   constexpr bool NARROW = G == 32;
   const uint32_t lds_r = (uint32_t)(l32 * 256 + (((l32 & 15) ^ (NARROW ? j : 4 * j)) << 4));
   const uint32_t woff = (uint32_t)l32 * wrow + 16u * WC * j;
-  const int col = min(wn0 + l32, N - 1);
+  const int col = min(wn0 + l32, N - 1), row = min(m0 + lane, M - 1);
 
   u32x4_t ra[2][AL], rb[2][WQ];
   float rs[2][NGU];
@@ -189,23 +206,32 @@ __global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
       rb[set][q] = buf_load16(
           rw, u < u1 ? woff + (uint32_t)(k0 * BITS / 8) + 32u * WC * (q / WC) + 16u * (q % WC) : kOob);
 #pragma unroll
-    for (int g = 0; g < NGU; ++g)
-      rs[set][g] = a.st[(int64_t)min(u * NGU + g, ng - 1) * N + col];
+    for (int g = 0; g < NGU; ++g) {
+      const int64_t gi = (int64_t)min(u, u1 - 1) * NGU + g;
+      rs[set][g] = a.st[gi * N + col];
+    }
   };
 
-  f32x16_t acc[2] = {f32x16_t{}, f32x16_t{}}, tmp[2];
+  f32x32_t acc = f32x32_t{};
+  f32x16_t tmp[2];
 
   auto body = [&](int u, auto stc) {
     constexpr int st = decltype(stc)::value;
     __builtin_amdgcn_sched_barrier(0);
     uint32_t wc[4 * WQ];
-    float sv[NGU];
+    float sv[NGU], bv[NGU], xv[NGU];
 #pragma unroll
     for (int q = 0; q < WQ; ++q)
 #pragma unroll
       for (int e = 0; e < 4; ++e) wc[4 * q + e] = rb[st][q][e];
 #pragma unroll
-    for (int g = 0; g < NGU; ++g) sv[g] = rs[st][g];
+    for (int g = 0; g < NGU; ++g) {
+      sv[g] = rs[st][g];
+      bv[g] = a.bt[(int64_t)(u * NGU + g) * N + col];
+      xv[g] = a.xs[(int64_t)(u * NGU + g) * M + row];
+    }
+    // (the bias operands of this unit before the next loads: waits count in order)
+    __builtin_amdgcn_sched_barrier(0);
     load(u + 2, st);
     if constexpr (NARROW) {
       // lane half j holds chunks 4j..4j+3 of each half; trade the upper half of
@@ -243,7 +269,9 @@ __global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
 #pragma unroll
           for (int x = 0; x < 2; ++x)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[x][e] = fmaf(sv[g], tmp[x][e], acc[x][e]);
+            for (int e = 0; e < 16; ++e) acc[16 * x + e] = fmaf(sv[g], tmp[x][e], acc[16 * x + e]);
+          // the group's bias part: two blocks of 32 rows, one k
+          acc = __builtin_amdgcn_mfma_f32_32x32x1f32(xv[g], bv[g], acc, 0, 0, 0);
         }
       }
     // slot st^1 was last read in unit u-1, before the barrier that ended it
@@ -266,40 +294,19 @@ __global__ __launch_bounds__(256, 2) void affine_gemm_kernel(AffGemmArgs a) {
   }
   if (u < u1) body(u, std::integral_constant<int, 0>{});
 
-  // bias part over this piece's groups, two per fp32 MFMA (k = lane half):
-  // four pairs' loads in flight
-  const int g1 = min(u1 * NGU, ng);
-  const int row0 = min(m0 + l32, M - 1), row1 = min(m0 + 32 + l32, M - 1);
-  for (int g = u0 * NGU; g < g1; g += 8) {
-    float xv[4][2], bv[4];
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const int gi = g + 2 * p + j, gc = min(gi, ng - 1);
-      const bool live = gi < g1;
-      xv[p][0] = a.xs[(int64_t)gc * M + row0];
-      xv[p][1] = a.xs[(int64_t)gc * M + row1];
-      bv[p] = a.bt[(int64_t)gc * N + col];
-      if (!live) xv[p][0] = xv[p][1] = bv[p] = 0.0f;
-    }
-#pragma unroll
-    for (int p = 0; p < 4; ++p)
-#pragma unroll
-      for (int x = 0; x < 2; ++x)
-        acc[x] = __builtin_amdgcn_mfma_f32_32x32x2f32(xv[p][x], bv[p], acc[x], 0, 0, 0);
-  }
-
   const bool split = a.S > 1;
   float* part = a.part + (int64_t)piece * M * N;
 #pragma unroll
   for (int x = 0; x < 2; ++x)
+#pragma unroll
     for (int e = 0; e < 16; ++e) {
       const int gm = m0 + 32 * x + mfma32_row(lane, e), gn = wn0 + l32;
       if (gm < M && gn < N) {
         const int64_t idx = (int64_t)gm * N + gn;
         if (split)
-          part[idx] = acc[x][e];
+          part[idx] = acc[16 * x + e];
         else
-          store_out(a.y, idx, acc[x][e], a.y_dtype);
+          store_out(a.y, idx, acc[16 * x + e], a.y_dtype);
       }
     }
 }
@@ -351,7 +358,7 @@ int aff_pieces(int64_t M, int64_t N, int64_t K) {
 }
 
 AffLayout aff_layout(int64_t M, int64_t N, int64_t K, int G, int S) {
-  const size_t ng = (size_t)(K / G);
+  const size_t ng = (size_t)cdiv(K, kAffBK) * (kAffBK / G);  // whole units
   AffLayout l;
   l.st = 0;
   l.bt = round_up(ng * N * 4, 256);
@@ -396,7 +403,9 @@ int affine_gemm(const void* x, const uint32_t* w, const void* s, const void* b, 
   q.K = (int)K;
   q.G = G;
   q.s_dtype = sdt;
-  q.wblocks = (int)(cdiv(N, 64) * cdiv(K / G, 32));
+  q.ngp = (int)cdiv(K, kAffBK) * (kAffBK / G);
+  q.centre = (float)(1 << (bits - 1));
+  q.wblocks = (int)(cdiv(N, 64) * cdiv(q.ngp, 32));
   const dim3 pg((unsigned)(q.wblocks + cdiv(M * (K / 8), 256)));
   if (xdt == SPARKQ_BF16)
     hipLaunchKernelGGL(affine_prep_kernel<BF16>, pg, dim3(256), 0, st, q);

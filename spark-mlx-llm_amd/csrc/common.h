@@ -81,8 +81,12 @@ typedef _Float16 f16x2_t __attribute__((ext_vector_type(2)));
 // packed 16-bit pairs (OFFSET+q[2i], OFFSET+q[2i+1]), i = 0..3, in natural k
 // order: a byte permute pulls code 2i from w and code 2i+1 from w>>4 into the
 // low nibble of each half, and one and-or masks the nibble under MAGIC.
+// (exact_f16_pair removes the fp16 magic 1024, and C more for codes centred
+// at C: whole numbers below 2048, so the difference is exact.)
+template <int C = 0>
 __device__ __forceinline__ uint32_t exact_f16_pair(uint32_t r) {
-  const f16x2_t v = __builtin_bit_cast(f16x2_t, r) - f16x2_t{(_Float16)1024.0f, (_Float16)1024.0f};
+  constexpr _Float16 off = (_Float16)(1024.0f + C);
+  const f16x2_t v = __builtin_bit_cast(f16x2_t, r) - f16x2_t{off, off};
   return __builtin_bit_cast(uint32_t, v);
 }
 
@@ -104,8 +108,9 @@ __device__ __forceinline__ DecodeConsts decode_consts() {
   return DecodeConsts{vgpr_const(0x000F000Fu), vgpr_const(T::MAGIC)};
 }
 
-template <typename T>
+template <typename T, int C = 0>
 __device__ __forceinline__ u32x4_t decode_w4(uint32_t w, DecodeConsts c) {
+  static_assert(C == 0 || T::kExactDecode, "only an exact decode can be centred");
   const uint32_t ws = w >> 4;
   u32x4_t r;
   r.x = (__builtin_amdgcn_perm(ws, w, 0x0C040C00u) & c.mask) | c.magic;
@@ -113,10 +118,10 @@ __device__ __forceinline__ u32x4_t decode_w4(uint32_t w, DecodeConsts c) {
   r.z = (__builtin_amdgcn_perm(ws, w, 0x0C060C02u) & c.mask) | c.magic;
   r.w = (__builtin_amdgcn_perm(ws, w, 0x0C070C03u) & c.mask) | c.magic;
   if constexpr (T::kExactDecode) {
-    r.x = exact_f16_pair(r.x);
-    r.y = exact_f16_pair(r.y);
-    r.z = exact_f16_pair(r.z);
-    r.w = exact_f16_pair(r.w);
+    r.x = exact_f16_pair<C>(r.x);
+    r.y = exact_f16_pair<C>(r.y);
+    r.z = exact_f16_pair<C>(r.z);
+    r.w = exact_f16_pair<C>(r.w);
   }
   return r;
 }

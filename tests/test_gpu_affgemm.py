@@ -70,3 +70,39 @@ def test_w8_prefill(gpu, m, n, k, g, dtype, sdtype, s, monkeypatch):
     monkeypatch.setenv("SPARKQ_W8AFF_GEMM_FROM", "1000000")
     z = sparkq.affine_quantized_matmul(*args, group_size=g, bits=8, out_dtype=torch.float32)
     assert rel_l2(y.cpu().numpy(), z.cpu().numpy()) <= 1e-5
+
+
+def _shifted(x, dtype, mean):
+    return o.round16(o.bits_to_f32(x, dtype) + np.float32(mean), dtype)
+
+
+@pytest.mark.parametrize("mean", [0.0, 1.0])
+@pytest.mark.parametrize("bits,m,n,k,g,dtype,sdtype,s", [
+    (4, 40, 128, 9728, 32, o.F16, o.F16, 1), (4, 64, 200, 9728, 64, o.F16, o.F16, 3),
+    (4, 33, 130, 9728, 128, o.F16, o.F16, 0), (4, 96, 256, 2624, 64, o.F16, o.F16, 1),
+    (8, 1, 512, 9728, 64, o.BF16, o.F32, 1), (8, 40, 128, 9728, 64, o.BF16, o.F32, 1),
+    (8, 64, 256, 2560, 64, o.BF16, o.BF16, 3), (8, 64, 200, 9728, 128, o.F16, o.F16, 1),
+    (8, 40, 130, 9728, 32, o.F16, o.F16, 1), (8, 33, 128, 2592, 32, o.BF16, o.F32, 0),
+])
+def test_error_over_long_rows(gpu, bits, m, n, k, g, dtype, sdtype, s, mean, monkeypatch):
+    """Long rows, and activations of mean 1, where the scale and bias parts
+    cancel. Each group rounds the running sum twice, by at most 2^-24 of it;
+    2 K/G roundings add in quadrature."""
+    import sparkq
+
+    print(f"[case] affgemm err w{bits} m={m} n={n} k={k} g={g} mean={mean}", flush=True)
+    _force(monkeypatch, s)
+    if bits == 4:
+        x, words, sc, b = w4_problem(m, n, k, g, dtype, seed=m + n)
+    else:
+        x, words, sc, b = _problem(m, n, k, g, dtype, sdtype, seed=m + n)
+    x = _shifted(x, dtype, mean)
+    ref = (o.w4a16_matmul(x, words, sc, b, g, dtype) if bits == 4
+           else o.w8_affine_matmul(x, words, sc, b, g, dtype, sdtype))
+    y = sparkq.affine_quantized_matmul(up16(x, dtype, gpu), up32(words, gpu),
+                                       _dev_scales(sc, sdtype, gpu), _dev_scales(b, sdtype, gpu),
+                                       group_size=g, bits=bits, out_dtype=torch.float32)
+    rel = rel_l2(y.cpu().numpy(), ref)
+    bound = (2 * k / g) ** 0.5 * 2.0 ** -24
+    print(f"rel {rel:.2e} bound {bound:.2e}", flush=True)
+    assert rel <= bound
