@@ -145,6 +145,8 @@ def call(name: str, *args, device: Optional[torch.device] = None) -> None:
 
 
 _WS: dict = {}
+_OUTGROWN: list = []  # replaced buffers: a captured graph may hold their addresses
+_WS_LOCK = threading.Lock()
 
 
 def workspace_buffer(device: torch.device, nbytes: int, kind: str) -> torch.Tensor:
@@ -157,12 +159,23 @@ def workspace(device: torch.device, nbytes: int, kind: str):
     """Scratch buffer per (device, stream, entry-point kind). Reuse is safe
     because every user enqueues on that same stream. Buffers start zeroed:
     split-K entry points keep tile counters at the front of their workspace,
-    which must be zero before the first call (every call leaves them zero)."""
+    which must be zero before the first call (every call leaves them zero).
+
+    A buffer that a larger call outgrows stays allocated: a HIP graph captured
+    on the stream replays with its address. Each is at least twice the one
+    before, so those kept are together smaller than the one in use."""
     if nbytes <= 0:
         return None, 0
     key = (device.index, _raw_stream(device), kind)
     buf = _WS.get(key)
     if buf is None or buf.numel() < nbytes:
-        buf = torch.zeros(max(nbytes, 1 << 20), dtype=torch.uint8, device=device)
-        _WS[key] = buf
+        with _WS_LOCK:
+            buf = _WS.get(key)
+            if buf is None or buf.numel() < nbytes:
+                size = max(nbytes, 1 << 20)
+                if buf is not None:
+                    size = max(size, 2 * buf.numel())
+                    _OUTGROWN.append(buf)
+                buf = torch.zeros(size, dtype=torch.uint8, device=device)
+                _WS[key] = buf
     return ctypes.c_void_p(buf.data_ptr()), buf.numel()
