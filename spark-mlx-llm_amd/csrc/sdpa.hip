@@ -578,7 +578,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void sdpa_prefill_kernel(Sdp
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
   int bx, by;
-  xcd_grid_item(a.xcd != 0, bx, by);
+  xcd_grid_item(a.xcd, bx, by);
   const int b = by / a.Hkv, kh = by - b * a.Hkv;
   const int R = a.L * GQA;                     // query rows (position, head) of this KV head
   // the wave's first row; under the causal mask the later (longer) row
@@ -896,7 +896,14 @@ __device__ __forceinline__ float sum_rows4(float v) {
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
-template <int D, typename T, bool SPLIT>
+// SPLIT: a tile's context in chunks, merged by the last of its workgroups.
+// OWN: the merge takes that workgroup's own sums from its registers; the
+// branch for it keeps the loads of one chunk from overlapping the next one's.
+// Us per call without / with it (causal, 16/4 heads of 256 and 64, 32/8 of
+// 128): two chunks, D=256 L = N = 1500 100 / 75, D=128 L = N = 512 36 / 23;
+// eight or four, D=256 L=64 N=4096 62 / 72, D=64 L = N = 500 14.9 / 18.3, but
+// D=128 L=64 N=4096 100 / 50 (its loads do not overlap either way).
+template <int D, typename T, bool SPLIT, bool OWN>
 __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void sdpa_prefill_affine_kernel(SdpaArgs a) {
   using LY = AffPrefillLds<D>;
   constexpr int NK = D / 32;                    // QK k chunks
@@ -910,7 +917,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void sdpa_prefill_affine_ker
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
   int bx, by;
-  xcd_grid_item(a.xcd != 0, bx, by);
+  xcd_grid_item(a.xcd, bx, by);
   const int b = by / a.Hkv, kh = by - b * a.Hkv;
   const int gqa = a.Hq / a.Hkv;
   const int R = a.L * gqa;  // (position, head) rows of this KV head
@@ -1174,21 +1181,21 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void sdpa_prefill_affine_ker
       float mm = kNegInf;
       for (int c = 0; c < S; ++c) mm = fmaxf(mm, splitk_load(a.pm + (pbase + c) * 128 + rrow));
       float z = 0.0f;
-      f32x4_t own[NJ];
+      f32x4_t own[OWN ? NJ : 1];
 #pragma unroll
       for (int j = 0; j < NJ; ++j) {
-        own[j] = acc[rt][j];
+        if (OWN) own[OWN ? j : 0] = acc[rt][j];
         acc[rt][j] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
       }
       for (int c = 0; c < S; ++c) {
         const float mc = splitk_load(a.pm + (pbase + c) * 128 + rrow);
         const float w = exp2_guarded(mc - mm, mc != kNegInf);
         z = fmaf(splitk_load(a.pz + (pbase + c) * 128 + rrow), w, z);
-        if (c == chunk) {  // this workgroup's own chunk, from its registers
+        if (OWN && c == chunk) {  // this workgroup's own chunk, from its registers
 #pragma unroll
           for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[rt][j][r] = fmaf(own[j][r], w, acc[rt][j][r]);
+            for (int r = 0; r < 4; ++r) acc[rt][j][r] = fmaf(own[OWN ? j : 0][r], w, acc[rt][j][r]);
           continue;
         }
 #pragma unroll
@@ -1746,7 +1753,8 @@ int int8kv_sdpa_prefill(const void* q, const void* kc, const void* ks, const voi
   // the row tiles of one (sequence, KV head) on one XCD, sharing its L2 for
   // the K/V blocks every wave re-reads (B=1 causal, 32/8 heads, D=128: L=N=2048
   // 185 -> 246 TFLOP/s; L=512 N=4096 unchanged)
-  a.xcd = !env_int("SPARKQ_PREFILL_NO_XCD", 0);
+  // Dealt: L=N=2048 16/4 heads of 256 220 -> 161 us, of 64 73 -> 60
+  a.xcd = env_int("SPARKQ_PREFILL_NO_XCD", 0) ? kXcdNone : kXcdDealt;
   const int gqa = (int)(Hq / Hkv);
   dim3 grid((unsigned)cdiv(L * gqa, 64), (unsigned)(B * Hkv));
   if (D == 64)
@@ -1758,19 +1766,21 @@ int int8kv_sdpa_prefill(const void* q, const void* kc, const void* ks, const voi
   return check_launch("sdpa_prefill_kernel");
 }
 
-template <int D, bool SPLIT>
+template <int D, bool SPLIT, bool OWN>
 static void launch_prefill_affine_s(const SdpaArgs& a, int qdt, dim3 grid, hipStream_t st) {
   if (qdt == SPARKQ_BF16)
-    hipLaunchKernelGGL((sdpa_prefill_affine_kernel<D, BF16, SPLIT>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((sdpa_prefill_affine_kernel<D, BF16, SPLIT, OWN>), grid, dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((sdpa_prefill_affine_kernel<D, F16, SPLIT>), grid, dim3(256), 0, st, a);
+    hipLaunchKernelGGL((sdpa_prefill_affine_kernel<D, F16, SPLIT, OWN>), grid, dim3(256), 0, st, a);
 }
 template <int D>
 static void launch_prefill_affine_d(const SdpaArgs& a, int qdt, dim3 grid, hipStream_t st) {
-  if (a.S > 1)
-    launch_prefill_affine_s<D, true>(a, qdt, grid, st);
-  else
-    launch_prefill_affine_s<D, false>(a, qdt, grid, st);
+  if (a.S <= 1)
+    launch_prefill_affine_s<D, false, false>(a, qdt, grid, st);
+  else if (D == 128 || a.S == 2)
+    launch_prefill_affine_s<D, true, true>(a, qdt, grid, st);
+  else if constexpr (D != 128)
+    launch_prefill_affine_s<D, true, false>(a, qdt, grid, st);
 }
 
 // Launch plan of the affine prefill: causal row tiles are paired when the
@@ -1860,8 +1870,15 @@ int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, co
   a.tps = (int)N;
   a.scale_log2 = scale * 1.4426950408889634f;
   // XCD-grouped work order (L=512 N=4096: D=128 275 -> 286, D=256 332 -> 344
-  // TFLOP/s; L=N=2048 unchanged)
-  a.xcd = !env_int("SPARKQ_PREFILL_NO_XCD", 0);
+  // TFLOP/s; L=N=2048 unchanged). Causal tiles at head dim 256, one workgroup
+  // per CU, are dealt where they need more than one round (16/4 heads, us with
+  // runs / dealt: L=N=1500 in two chunks 102 / 74, L=N=3072 in two 273 / 215); in
+  // one round, and at two workgroups per CU, runs are level or better (L=N=512
+  // D=256 31.8 / 33.0, D=128 23.4 / 24.4, L=512 N=4096 D=128 57.4 / 60.4).
+  const int64_t ntiles = cdiv(L * (Hq / Hkv), 128);
+  const dim3 grid((unsigned)(plan.pair ? cdiv(ntiles, 2) : ntiles * plan.S), (unsigned)(B * Hkv));
+  a.xcd = D == 256 && causal && (int64_t)grid.x * grid.y > device_cus() ? kXcdDealt : kXcdRuns;
+  if (env_int("SPARKQ_PREFILL_NO_XCD", 0)) a.xcd = kXcdNone;
   if (plan.S > 1) {
     unsigned char* base = reinterpret_cast<unsigned char*>(ws);
     const size_t rows = round_up((size_t)plan.ntiles_all * plan.S * 128 * 4, 256);
@@ -1870,8 +1887,6 @@ int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, co
     a.pz = reinterpret_cast<float*>(base + kCounterBytes + rows);
     a.pacc = reinterpret_cast<float*>(base + kCounterBytes + 2 * rows);
   }
-  const int64_t ntiles = cdiv(L * (Hq / Hkv), 128);
-  dim3 grid((unsigned)(plan.pair ? cdiv(ntiles, 2) : ntiles * plan.S), (unsigned)(B * Hkv));
   if (D == 64)
     launch_prefill_affine_d<64>(a, qdt, grid, st);
   else if (D == 128)

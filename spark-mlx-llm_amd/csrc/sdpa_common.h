@@ -34,24 +34,25 @@ struct SdpaArgs {
 };
 
 // Workgroup (x, y) of a 2-D grid is dispatched as item y * gx + x and runs
-// on XCD item % 8. With xcd set, the item order is regrouped so that each XCD
+// on XCD item % 8. kXcdRuns: the item order is regrouped so that each XCD
 // takes a contiguous chunk of the (y, x) order: the row tiles of one
 // (sequence, KV head) share an XCD's L2 for their K/V blocks, and within a
 // chunk the items keep their relative order (the longest causal tiles still
-// start first). Where k XCDs share one (sequence, KV head), each takes every
-// k-th of its items: contiguous runs would leave the long causal tiles to one
-// XCD and the short ones to another. A bijection on the grid; a grid of a size
-// not divisible by 8 keeps its order.
-__device__ __forceinline__ void xcd_grid_item(bool xcd, int& x, int& y) {
+// start first). kXcdDealt: where k XCDs share one (sequence, KV head), each
+// takes every k-th of its items; contiguous runs leave the long causal tiles
+// to one XCD and the short ones to another. A bijection on the grid; a grid of
+// a size not divisible by 8 keeps its order.
+constexpr int kXcdNone = 0, kXcdRuns = 1, kXcdDealt = 2;
+__device__ __forceinline__ void xcd_grid_item(int xcd, int& x, int& y) {
   x = (int)blockIdx.x;
   y = (int)blockIdx.y;
   const int gx = (int)gridDim.x, T = gx * (int)gridDim.y;
-  if (!xcd || (T & 7) != 0) return;
+  if (xcd == kXcdNone || (T & 7) != 0) return;
   const int id = y * gx + x, m = T >> 3, v = (id & 7) * m + (id >> 3);
   y = v / gx;
   x = v - y * gx;
   const int k = gx / m;
-  if (k > 1 && k * m == gx) x = x % m * k + x / m;
+  if (xcd == kXcdDealt && k > 1 && k * m == gx) x = x % m * k + x / m;
 }
 
 constexpr float kNegInf = -__builtin_huge_valf();

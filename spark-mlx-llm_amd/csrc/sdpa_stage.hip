@@ -125,7 +125,7 @@ __global__ __launch_bounds__(256, D <= 128 ? 2 : 1) void sdpa_stage_kernel(GenSd
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n16 = lane & 15, grp = lane >> 4;
   int bx, by;
-  xcd_grid_item(true, bx, by);
+  xcd_grid_item(kXcdDealt, bx, by);
   const int b = by / a.Hkv, kh = by - b * a.Hkv;
   const int gqa = a.Hq / a.Hkv;
   const int R = a.L * gqa;
