@@ -376,7 +376,8 @@ int sparkq_int8kv_sdpa_prefill(const void* q, const void* k_codes,
  * same launch: that needs the workspace of
  * sparkq_int8kv_sdpa_prefill_affine_workspace_bytes (0 when no split; tile
  * counters in its first 16384 bytes, zero before the first call and left
- * zero, then partials). Calls that share a workspace must not overlap.
+ * zero, then partials). Causal prompts at D=256 may also be split for balance;
+ * those run unsplit without the workspace. Calls that share a workspace must not overlap.
  * Replaces the L > 1 branch of int8_quantized_sdpa
  * (X/spark_mlx_ext/int8_quantized_sdpa.py:236-245) and its kernel
  * spark_affine_u8_sdpa_prefill (X/spark_mlx_ext/int8_quantized_sdpa_prefill.py:

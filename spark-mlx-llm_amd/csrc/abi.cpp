@@ -60,7 +60,7 @@ int int8kv_sdpa_prefill(const void* q, const void* kc, const void* ks, const voi
                         int64_t N, int64_t D, int causal, int qdt, int odt, float scale,
                         const int64_t* strides, hipStream_t st);
 size_t int8kv_sdpa_prefill_affine_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
-                                            int64_t D, int causal);
+                                            int64_t N, int64_t D, int causal);
 int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, const void* kb,
                                const void* vc, const void* vs, const void* vb, void* out,
                                int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
@@ -556,9 +556,8 @@ int sparkq_int8kv_sdpa_prefill_affine(const void* q, const void* k_packed, const
 size_t sparkq_int8kv_sdpa_prefill_affine_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv,
                                                          int64_t L, int64_t N, int64_t D,
                                                          int causal) {
-  (void)N;
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || D <= 0 || Hq % Hkv) return 0;
-  return int8kv_sdpa_prefill_affine_workspace(B, Hq, Hkv, L, D, causal);
+  return int8kv_sdpa_prefill_affine_workspace(B, Hq, Hkv, L, N, D, causal);
 }
 
 int sparkq_kv_append(const void* x, void* codes, void* scales, void* biases, int64_t B,

@@ -1787,19 +1787,39 @@ static void launch_prefill_affine_d(const SdpaArgs& a, int qdt, dim3 grid, hipSt
 // paired grid still has a workgroup for every CU (D <= 128); a grid short of
 // one workgroup per CU splits each tile's blocks over S <= 8 workgroups,
 // merged in the same launch through the workspace (tile counters, then the
-// per-chunk maxima, sums and accumulators). At head dim 256, where a workgroup
-// has a CU to itself, one round of causal tiles lasts as long as its longest
-// one: from one to two tiles per CU each is split in two, whose halves, longest
-// first, even out (16/4 heads, L = N = 2048: 142 us -> 115), as long as the
-// context is at most half as long again as the queries (N is known at the
-// launch only); with longer ones the tiles are nearly alike.
+// per-chunk maxima, sums and accumulators).
 struct AffPrefillPlan {
   int pair, S;
-  bool halves;
+  bool halves;  // S = 2 for balance: not needed, so a call without the workspace runs whole tiles
   int64_t ntiles_all;
   size_t bytes;
 };
-static AffPrefillPlan plan_prefill_affine(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
+// Causal tiles at head dim 256, where a workgroup has a CU to itself: with
+// little more than one tile per CU the prompt lasts as long as its longest
+// tile, twice the average, and each tile in two halves, longest first, evens
+// that out. The halves cost a merge and a second start per CU, 20 to 40 us
+// together, and a half saves about 0.03 us per query token: from 2048 tokens
+// on it pays. Whole tiles -> halves, us, 16/4 heads unless stated:
+//   one tile per CU       L=N=2048 137 -> 113, 1024 75.5 -> 74.5, 512 (four
+//                         sequences) 45 -> 58, 256 (eight) 30 -> 53, 8/2 4096 257 -> 176
+//   9/8 tiles per CU      L=2304 151 -> 148, 8/2 L=4416 276 -> 220, L=1152 (two) 84 -> 102
+//   19/16 and more        L=2432 159 -> 160, 2560 168 -> 172, 3072 198 -> 219
+// A grid of whole tiles that is no multiple of 8 is not dealt over the XCDs,
+// and where the last (sequence, KV head) starts after a full round its longest
+// tiles run on: L=3104 268 -> 225, 3616 331 -> 281, 4064 438 -> 340.
+// Both need a dealing that evens out (the XCDs a multiple of the (sequence, KV
+// head) pairs or the other way round): 20/5 L=2688 245 -> 281. The gain does
+// not depend on N (L=2048, N=3072 197 -> 172, 4096 259 -> 235), but its share
+// does, and the partials take 67 MB: up to 3/2 L.
+static bool prefill_halves(int64_t BH, int64_t tiles, int64_t L, int64_t N, int64_t D, int causal) {
+  const int64_t cus = device_cus();
+  if (D != 256 || !causal || tiles < cus || tiles >= 2 * cus || 2 * N > 3 * L) return false;
+  if (env_int("SPARKQ_PREFILL_NO_HALVES", 0)) return false;
+  if (env_int("SPARKQ_PREFILL_HALVES", 0)) return true;
+  if (L < 2048 || (8 % BH != 0 && BH % 8 != 0)) return false;
+  return tiles <= cus + cus / 8 || (tiles % 8 != 0 && tiles - tiles / BH >= cus);
+}
+static AffPrefillPlan plan_prefill_affine(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
                                           int64_t D, int causal) {
   AffPrefillPlan p{};
   const int64_t ntiles = cdiv(L * (Hq / Hkv), 128);
@@ -1812,8 +1832,8 @@ static AffPrefillPlan plan_prefill_affine(int64_t B, int64_t Hq, int64_t Hkv, in
   }();
   if (!p.pair && p.ntiles_all < target && p.ntiles_all <= (int64_t)(kCounterBytes / 4))
     p.S = (int)std::min<int64_t>(8, cdiv(target, p.ntiles_all));
-  else if (D == 256 && causal && p.ntiles_all >= 256 && p.ntiles_all < 512 &&
-           !env_int("SPARKQ_PREFILL_NO_HALVES", 0))
+  else if (p.ntiles_all <= (int64_t)(kCounterBytes / 4) &&
+           prefill_halves(B * Hkv, p.ntiles_all, L, N, D, causal))
     p.S = 2, p.halves = true;
   p.bytes = p.S > 1 ? kCounterBytes + round_up((size_t)p.ntiles_all * p.S * 128 * 4, 256) * 2 +
                           (size_t)p.ntiles_all * p.S * 128 * D * 4
@@ -1822,8 +1842,8 @@ static AffPrefillPlan plan_prefill_affine(int64_t B, int64_t Hq, int64_t Hkv, in
 }
 
 size_t int8kv_sdpa_prefill_affine_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
-                                            int64_t D, int causal) {
-  return plan_prefill_affine(B, Hq, Hkv, L, D, causal).bytes;
+                                            int64_t N, int64_t D, int causal) {
+  return plan_prefill_affine(B, Hq, Hkv, L, N, D, causal).bytes;
 }
 
 int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, const void* kb,
@@ -1831,8 +1851,8 @@ int int8kv_sdpa_prefill_affine(const void* q, const void* kc, const void* ks, co
                                int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
                                int64_t D, int G, int causal, int qdt, int odt, float scale,
                                const int64_t* strides, void* ws, size_t wsb, hipStream_t st) {
-  AffPrefillPlan plan = plan_prefill_affine(B, Hq, Hkv, L, D, causal);
-  if (plan.halves && 2 * N > 3 * L) plan.S = 1;
+  AffPrefillPlan plan = plan_prefill_affine(B, Hq, Hkv, L, N, D, causal);
+  if (plan.halves && (ws == nullptr || wsb < plan.bytes)) plan.S = 1;
   if (plan.S > 1 && (ws == nullptr || wsb < plan.bytes))
     return set_error(SPARKQ_ERR_WORKSPACE, "int8kv_sdpa_prefill_affine: workspace too small");
   SdpaArgs a{};
