@@ -513,11 +513,16 @@ int sparkq_rope(const void* x, void* out, int64_t rows, int64_t L, int64_t D, in
  * nothing averages all values. Scores, softmax and output run in fp32 (the
  * reference's staged form rounds q*scale, the scores and the weights to the
  * query dtype). A long context is split over several workgroups and merged
- * by a second launch; the workspace (sparkq_quantized_sdpa_workspace_bytes,
- * 0 without a split) holds the partials.
+ * by a second launch; the workspace (sparkq_quantized_sdpa_workspace_bytes:
+ * enough for every query type and key head dim;
+ * sparkq_quantized_sdpa_call_workspace_bytes: for these; 0 without a split)
+ * holds the partials. It needs no initial value.
  * ---------------------------------------------------------------------- */
 size_t sparkq_quantized_sdpa_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv,
                                              int64_t L, int64_t N, int64_t Dv);
+size_t sparkq_quantized_sdpa_call_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv,
+                                                  int64_t L, int64_t N, int64_t D,
+                                                  int64_t Dv, int q_dtype);
 int sparkq_quantized_sdpa(const void* q, const void* k_packed, const void* k_scales,
                           const void* k_biases, const void* v_packed,
                           const void* v_scales, const void* v_biases,

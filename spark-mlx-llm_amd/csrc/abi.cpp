@@ -89,8 +89,8 @@ int rms_norm(const void* x, const void* xres, const void* w, float eps, void* hi
 int attention_gate(const void* x, const void* attn, const void* gw, void* out, void* gate_out,
                    int64_t B, int64_t L, int64_t H, int64_t D, int64_t K, int dt,
                    hipStream_t st);
-size_t sdpa_gen_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
-                          int64_t Dv);
+size_t sdpa_gen_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N, int64_t D,
+                          int64_t Dv, int qdt);
 int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, const void* vp,
                  const void* vs, const void* vb, const void* mask, int mask_kind,
                  int mask_dtype, const int64_t* mask_strides, void* out, int64_t B, int64_t Hq,
@@ -796,7 +796,12 @@ int sparkq_attention_gate(const void* x, const void* attn, const void* gate_w, v
 
 size_t sparkq_quantized_sdpa_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
                                              int64_t N, int64_t Dv) {
-  return sdpa_gen_workspace(B, Hq, Hkv, L, N, Dv);
+  return sdpa_gen_workspace(B, Hq, Hkv, L, N, 0, Dv, 0);
+}
+
+size_t sparkq_quantized_sdpa_call_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t L,
+                                                  int64_t N, int64_t D, int64_t Dv, int q_dtype) {
+  return D > 0 ? sdpa_gen_workspace(B, Hq, Hkv, L, N, D, Dv, q_dtype) : 0;
 }
 
 int sparkq_quantized_sdpa(const void* q, const void* k_packed, const void* k_scales,

@@ -38,8 +38,9 @@ struct GenSdpaArgs {
 
 constexpr int kMaskNone = 0, kMaskCausal = 1, kMaskBool = 2, kMaskAdd = 3;
 
-// sdpa_stage.hip: whether the matrix-core kernel takes the call, its context
-// splits, its launch, and the merge of its partials
+// sdpa_stage.hip: whether the matrix-core kernel takes the types and head dims,
+// and the call, its context splits and its launch
+bool sdpa_stage_dims(int qdt, int64_t D, int64_t Dv);
 bool sdpa_stage_ok(const GenSdpaArgs& a);
 int sdpa_stage_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N);
 int launch_sdpa_stage(const GenSdpaArgs& a, hipStream_t st);

@@ -427,16 +427,17 @@ static size_t gen_partial_bytes(size_t rows, int64_t S, int64_t Dv) {
   return round_up(rows * S * 4, 256) * 2 + round_up(rows * S * Dv * 4, 256);
 }
 
-// covers both kernels (the query type and the key head dim, which choose
-// between them, are not known here)
-size_t sdpa_gen_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N,
-                          int64_t Dv) {
+// The partials of one call. Whether sdpa_stage_kernel takes it depends on the
+// alignment of q and out too, so a call of its types and head dims is given the
+// larger of both kernels' needs; D = 0: any type and key head dim.
+size_t sdpa_gen_workspace(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N, int64_t D,
+                          int64_t Dv, int qdt) {
   if (B <= 0 || Hq <= 0 || Hkv <= 0 || L <= 0 || N <= 0 || Dv <= 0 || Hq % Hkv) return 0;
   int RC, nch, S;
   int64_t tps;
   gen_plan(B, Hq, Hkv, L, N, &RC, &nch, &S, &tps);
-  const size_t rows = (size_t)B * Hq * L;
-  return gen_partial_bytes(rows, std::max(S, sdpa_stage_splits(B, Hq, Hkv, L, N)), Dv);
+  if (D == 0 || sdpa_stage_dims(qdt, D, Dv)) S = std::max(S, sdpa_stage_splits(B, Hq, Hkv, L, N));
+  return gen_partial_bytes((size_t)B * Hq * L, S, Dv);
 }
 
 int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, const void* vp,
@@ -490,7 +491,17 @@ int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, 
   gen_plan(B, Hq, Hkv, L, N, &a.RC, &a.nch, &a.S, &tps);
   a.tps = (int)tps;
   const bool stage = sdpa_stage_ok(a);
-  if (stage) a.S = sdpa_stage_splits(B, Hq, Hkv, L, N);
+  const size_t rows = (size_t)B * Hq * L;
+  const size_t need = gen_partial_bytes(rows, a.S, Dv);
+  if (need > 0 && (ws == nullptr || wsb < need))
+    return set_error(SPARKQ_ERR_WORKSPACE,
+                     "quantized_sdpa needs a workspace of %zu bytes (got %zu)", need, wsb);
+  if (stage) {
+    // its splits fill the chip, and fewer do too: as many as fit a workspace
+    // that is smaller
+    a.S = sdpa_stage_splits(B, Hq, Hkv, L, N);
+    while (a.S > 1 && (ws == nullptr || wsb < gen_partial_bytes(rows, a.S, Dv))) --a.S;
+  }
   a.scale_log2 = scale * 1.4426950408889634f;
   // the reference fills masked scores with the lowest finite value of the
   // query dtype: any visible score outweighs it completely, and a row with
@@ -500,11 +511,6 @@ int sdpa_generic(const void* q, const void* kp, const void* ks, const void* kb, 
   a.masked = qdt == SPARKQ_F16 ? -65504.0f : qdt == SPARKQ_BF16 ? -3.38953139e38f
                                                                   : -3.40282347e38f;
   if (a.S > 1) {
-    const size_t need = gen_partial_bytes((size_t)B * Hq * L, a.S, Dv);
-    if (ws == nullptr || wsb < need)
-      return set_error(SPARKQ_ERR_WORKSPACE,
-                       "quantized_sdpa needs a workspace of %zu bytes (got %zu)", need, wsb);
-    const size_t rows = (size_t)B * Hq * L;
     unsigned char* p = static_cast<unsigned char*>(ws);
     a.pm = reinterpret_cast<float*>(p);
     a.pz = reinterpret_cast<float*>(p + round_up(rows * a.S * 4, 256));

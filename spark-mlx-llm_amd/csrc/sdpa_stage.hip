@@ -486,11 +486,16 @@ int sdpa_stage_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N) 
   return (int)std::min<int64_t>(S, 128);
 }
 
-// 16-bit queries, one head dim of 64/96/128/256, 16-byte aligned q and out and
-// a context whose byte offsets fit 31 bits; groups that divide the head dim.
+// 16-bit queries and one head dim of 64/96/128/256
+bool sdpa_stage_dims(int qdt, int64_t D, int64_t Dv) {
+  return (qdt == SPARKQ_BF16 || qdt == SPARKQ_F16) && D == Dv &&
+         (D == 64 || D == 96 || D == 128 || D == 256);
+}
+
+// ..., 16-byte aligned q and out and a context whose byte offsets fit 31 bits;
+// groups that divide the head dim.
 bool sdpa_stage_ok(const GenSdpaArgs& a) {
-  if (a.q_dtype != SPARKQ_BF16 && a.q_dtype != SPARKQ_F16) return false;
-  if (a.D != a.Dv || (a.D != 64 && a.D != 96 && a.D != 128 && a.D != 256)) return false;
+  if (!sdpa_stage_dims(a.q_dtype, a.D, a.Dv)) return false;
   if (!aligned(a.q, 16) || !aligned(a.out, 16)) return false;
   const int64_t lim = (int64_t)1 << 31;
   const int64_t n = (int64_t)a.N + 96;  // the loads run up to two blocks ahead

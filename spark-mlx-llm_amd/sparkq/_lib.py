@@ -74,6 +74,7 @@ SIGNATURES = {
     "sparkq_rms_norm": (I, [P, P, P, F, P, P, I64, I64, I, P]),
     "sparkq_attention_gate": (I, [P, P, P, P, P, I64, I64, I64, I64, I64, I, P]),
     "sparkq_quantized_sdpa_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I64]),
+    "sparkq_quantized_sdpa_call_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I64, I64, I]),
     "sparkq_quantized_sdpa": (I, [P, P, P, P, P, P, P, P, I, I, P, P, I64, I64, I64, I64, I64,
                                   I64, I64, I, I, I, I, F, P, P, SZ, P]),
 }

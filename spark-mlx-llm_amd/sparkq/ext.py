@@ -892,8 +892,9 @@ def _staged_attention(queries, keys, values, *, scale, group_size, bits, mask, o
     y = _out_buffer(out, (batch, heads, length, dv), out_dtype, queries.device)
     st = (ctypes.c_int64 * 12)(*(_kv_strides(kc, ks, 4) + _kv_strides(vc, vs, 4)))
     ws, wsb = _lib.workspace(queries.device,
-                             _lib.lib().sparkq_quantized_sdpa_workspace_bytes(
-                                 batch, heads, kv_heads, length, n, dv), "sdpa_staged")
+                             _lib.lib().sparkq_quantized_sdpa_call_workspace_bytes(
+                                 batch, heads, kv_heads, length, n, dim, dv,
+                                 _lib.dtype_code(queries.dtype)), "sdpa_staged")
     _lib.call("sparkq_quantized_sdpa", _ptr(q), _ptr(kc), _ptr(ks), _ptr(kb), _ptr(vc),
               _ptr(vs), _ptr(vb), _ptr(mask_t), kind, mdt, mstrides, _ptr(y), batch, heads,
               kv_heads, length, n, dim, dv, group_size, bits, _lib.dtype_code(queries.dtype),

@@ -80,3 +80,47 @@ def test_stage_kernel_matches_oracle(gpu, b, hq, hkv, length, n, d, g, bits, qdt
     qt = flat.view(qt.shape)
     rel = np.linalg.norm(attend(kt, vt).cpu().numpy() - ref) / np.linalg.norm(ref)
     assert rel <= 1e-5
+
+
+def test_stage_takes_a_smaller_workspace(gpu):
+    """A C caller may give less than the matrix-core kernel's splits use, down
+    to what the vector kernel needs (nothing here): it then runs fewer. Less
+    than that is refused."""
+    import ctypes
+
+    from sparkq import _lib
+
+    print("[case] stage with a small workspace", flush=True)
+    hq, hkv, length, n, d, g, bits = 32, 8, 200, 900, 128, 64, 4
+    (kt, _), (vt, _) = (_cache(gpu, 1, hkv, n, d, g, bits, o.BF16, i) for i in (0, 1))
+    qt = up16(o.randn16(4, 72, hq * length * d).reshape(1, hq, length, d), o.BF16, gpu)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    ng = d // g
+    strides = (ctypes.c_int64 * 12)(*(2 * [hkv * n * d // 2, n * d // 2, d // 2,
+                                           hkv * n * ng, n * ng, ng]))
+
+    def attend(nbytes, rows=length):
+        ws = torch.empty(nbytes, dtype=torch.uint8, device=gpu) if nbytes else None
+        y = torch.full((1, hq, rows, d), float("nan"), dtype=torch.float32, device=gpu)
+        q = qt[:, :, :rows].contiguous()
+        rc = _lib.lib().sparkq_quantized_sdpa(
+            ptr(q), *map(ptr, kt), *map(ptr, vt), None, 1, _lib.F32, None, ptr(y), 1, hq, hkv,
+            rows, n, d, d, g, bits, _lib.BF16, _lib.F32, d ** -0.5, strides,
+            ptr(ws) if nbytes else None, nbytes, _lib.stream_handle(gpu))
+        torch.cuda.synchronize()
+        return rc, y
+
+    query = _lib.lib().sparkq_quantized_sdpa_call_workspace_bytes
+    full = query(1, hq, hkv, length, n, d, d, _lib.BF16)
+    assert full > query(1, hq, hkv, length, n, d, d, _lib.F32) == 0
+    rc, ref = attend(full)
+    assert rc == 0
+    for nbytes in (full - 1, full // 2, 4096, 0):
+        rc, y = attend(nbytes)
+        assert rc == 0, (nbytes, _lib.lib().sparkq_last_error())
+        assert float((y - ref).norm()) <= 1e-5 * float(ref.norm()), nbytes
+    # one row: the vector kernel splits too, and its need is the least
+    least = query(1, hq, hkv, 1, n, d, d, _lib.F32)
+    assert least > 0
+    assert attend(least, 1)[0] == 0
+    assert attend(least - 1, 1)[0] == _lib.ERR_WORKSPACE

@@ -35,6 +35,21 @@ def test_outgrown_buffers_stay(host_buffers):
     assert sum(sizes[:-1]) < sizes[-1] == _lib.workspace(host_buffers, 1, "kind")[1]
 
 
+def test_attention_workspace_fits_the_call():
+    """fp32 queries and head dims of the vector kernel are not sized for the
+    matrix-core kernel's splits."""
+    lib = _lib.lib()
+    call, any_call = (lib.sparkq_quantized_sdpa_call_workspace_bytes,
+                      lib.sparkq_quantized_sdpa_workspace_bytes)
+    shape = (1, 32, 8, 512, 4096)
+    assert call(*shape, 128, 128, _lib.F32) == 0
+    assert call(*shape, 160, 160, _lib.BF16) == 0
+    assert call(*shape, 128, 64, _lib.BF16) == 0
+    assert call(*shape, 128, 128, _lib.BF16) == any_call(*shape, 128) > 0
+    assert call(1, 32, 8, 1, 4096, 128, 128, _lib.F32) > 0
+    assert call(0, 32, 8, 1, 4096, 128, 128, _lib.F32) == 0
+
+
 def _w4(gpu, m, n, k, g, seed):
     gen = torch.Generator().manual_seed(seed)
     x = torch.randn((m, k), generator=gen).to(torch.bfloat16).to(gpu)
