@@ -16,7 +16,7 @@ import torch
 
 __all__ = [
     "F32", "F16", "BF16", "KV_S8_F16SCALE", "KV_AFFINE_U8",
-    "lib", "library_path", "dtype_code", "call", "stream_handle", "workspace",
+    "lib", "library_path", "dtype_code", "call", "stream_handle", "workspace", "scratch",
     "SparkqError",
 ]
 
@@ -180,3 +180,12 @@ def workspace(device: torch.device, nbytes: int, kind: str):
                 buf = torch.zeros(size, dtype=torch.uint8, device=device)
                 _WS[key] = buf
     return ctypes.c_void_p(buf.data_ptr()), buf.numel()
+
+
+def scratch(device: torch.device, nbytes: int) -> Optional[torch.Tensor]:
+    """Workspace of one call, for entry points that need no initial value in it:
+    memory of the current stream from torch's allocator (of a graph's own pool
+    under capture), which the caller drops once the call is enqueued. A call of
+    several launches has its own, so that two threads that enqueue on one
+    stream, or two graphs captured on one, do not share partial results."""
+    return torch.empty(nbytes, dtype=torch.uint8, device=device) if nbytes > 0 else None

@@ -241,11 +241,11 @@ def _w8_affine_matmul(op, x, weight, scales, biases, group_size, out_dtype, out)
         return y.reshape(*lead, n)
     x2 = x.reshape(m, k).contiguous()
     weight, scales, biases = weight.contiguous(), scales.contiguous(), biases.contiguous()
-    ws, wsb = _lib.workspace(x.device, _lib.lib().sparkq_w8_affine_workspace_bytes(
-        m, n, k, group_size), "w8_affine")
+    need = _lib.lib().sparkq_w8_affine_workspace_bytes(m, n, k, group_size)
+    ws = _lib.scratch(x.device, need)
     _lib.call("sparkq_w8_affine_linear_ws", _ptr(x2), _ptr(weight), _ptr(scales), _ptr(biases),
               _ptr(y), m, n, k, group_size, _lib.dtype_code(x.dtype),
-              _lib.dtype_code(scales.dtype), _lib.dtype_code(out_dtype), ws, wsb,
+              _lib.dtype_code(scales.dtype), _lib.dtype_code(out_dtype), _ptr(ws), need,
               _lib.stream_handle(x.device), device=x.device)
     return y.reshape(*lead, n)
 
@@ -891,14 +891,13 @@ def _staged_attention(queries, keys, values, *, scale, group_size, bits, mask, o
     q = queries.contiguous()
     y = _out_buffer(out, (batch, heads, length, dv), out_dtype, queries.device)
     st = (ctypes.c_int64 * 12)(*(_kv_strides(kc, ks, 4) + _kv_strides(vc, vs, 4)))
-    ws, wsb = _lib.workspace(queries.device,
-                             _lib.lib().sparkq_quantized_sdpa_call_workspace_bytes(
-                                 batch, heads, kv_heads, length, n, dim, dv,
-                                 _lib.dtype_code(queries.dtype)), "sdpa_staged")
+    need = _lib.lib().sparkq_quantized_sdpa_call_workspace_bytes(
+        batch, heads, kv_heads, length, n, dim, dv, _lib.dtype_code(queries.dtype))
+    ws = _lib.scratch(queries.device, need)
     _lib.call("sparkq_quantized_sdpa", _ptr(q), _ptr(kc), _ptr(ks), _ptr(kb), _ptr(vc),
               _ptr(vs), _ptr(vb), _ptr(mask_t), kind, mdt, mstrides, _ptr(y), batch, heads,
               kv_heads, length, n, dim, dv, group_size, bits, _lib.dtype_code(queries.dtype),
-              _lib.dtype_code(out_dtype), float(scale), st, ws, wsb,
+              _lib.dtype_code(out_dtype), float(scale), st, _ptr(ws), need,
               _lib.stream_handle(queries.device), device=queries.device)
     return y
 

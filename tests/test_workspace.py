@@ -59,6 +59,98 @@ def _w4(gpu, m, n, k, g, seed):
     return x, w, s, b
 
 
+def _w8(gpu, m, n, k, g, seed):
+    x, w, s, b = _w4(gpu, m, n, k, g, seed)
+    return x, torch.cat([w, w.flip(0)], 1), s, b
+
+
+def test_calls_of_several_launches_share_no_scratch(monkeypatch):
+    """Groupwise 8-bit and staged attention calls ask the allocator each time:
+    two calls that are enqueued together hold different memory."""
+    from sparkq import ext
+
+    monkeypatch.setattr(_lib, "workspace", lambda *a: pytest.fail("shared workspace"))
+    monkeypatch.setattr(_lib, "stream_handle", lambda device: None)
+    monkeypatch.setattr(ext, "_require_device", lambda *a: None)
+    held, live = [], []
+
+    def scratch(device, nbytes):
+        assert nbytes > 0
+        live.append(torch.empty(nbytes, dtype=torch.uint8))
+        return live[-1]
+
+    def call(name, *args, device=None):
+        held.append([a for a in args if a == live[-1].data_ptr()])
+
+    monkeypatch.setattr(_lib, "scratch", scratch)
+    monkeypatch.setattr(_lib, "call", call)
+    cpu = torch.device("cpu")
+    for seed in (1, 2):
+        ext.affine_quantized_matmul(*_w8(cpu, 4, 256, 2560, 64, seed), group_size=64, bits=8)
+        kv = (torch.zeros((1, 8, 900, 16), dtype=torch.int32),
+              *(torch.zeros((1, 8, 900, 2), dtype=torch.bfloat16) for _ in range(2)))
+        q = torch.zeros((1, 32, 4, 128), dtype=torch.bfloat16)
+        ext.int8_quantized_sdpa(q, kv, kv, scale=1.0, group_size=64, bits=4, mask="causal")
+    assert all(len(h) == 1 for h in held) and len({h[0] for h in held}) == 4
+
+
+@pytest.mark.gpu
+def test_threads_on_one_stream(gpu):
+    """Two threads enqueue 8-bit calls on the same stream, interleaving their
+    launches as they like: each gets its own result."""
+    import threading
+
+    import sparkq
+
+    print("[case] two threads, one stream", flush=True)
+    problems = [_w8(gpu, m, 1024, 2560, 64, m) for m in (8, 9)]
+    call = lambda p: sparkq.affine_quantized_matmul(*p, group_size=64, bits=8)  # noqa: E731
+    refs = [call(p) for p in problems]
+    torch.cuda.synchronize()
+    bad = []
+
+    def work(i):
+        for _ in range(100):
+            outs = [call(problems[i]) for _ in range(4)]
+            if not all(torch.equal(y, refs[i]) for y in outs):
+                bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+
+
+@pytest.mark.gpu
+def test_two_graphs_on_one_capture_stream(gpu):
+    """Graphs captured on one stream replay on two streams at once."""
+    import sparkq
+
+    print("[case] two graphs replayed side by side", flush=True)
+    problems = [_w8(gpu, m, 1024, 2560, 64, m) for m in (8, 9)]
+    refs = [sparkq.affine_quantized_matmul(*p, group_size=64, bits=8) for p in problems]
+    outs = [torch.empty_like(r) for r in refs]
+    torch.cuda.synchronize()
+    side, graphs = torch.cuda.Stream(), []
+    for p, y in zip(problems, outs):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[-1], stream=side):
+            for _ in range(10):
+                sparkq.affine_quantized_matmul(*p, group_size=64, bits=8, out=y)
+    streams = [torch.cuda.Stream() for _ in graphs]
+    for replay in range(5):
+        for y in outs:
+            y.zero_()
+        torch.cuda.synchronize()
+        for graph, stream in zip(graphs, streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(y, r) for y, r in zip(outs, refs)), replay
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits", [4, 8])
 def test_graph_survives_a_larger_call(gpu, bits):
@@ -71,10 +163,7 @@ def test_graph_survives_a_larger_call(gpu, bits):
     g = 64
 
     def problem(m, n, k, seed):
-        x, w, s, b = _w4(gpu, m, n, k, g, seed)
-        if bits == 8:
-            w = torch.cat([w, w.flip(0)], 1)
-        return x, w, s, b
+        return (_w4 if bits == 4 else _w8)(gpu, m, n, k, g, seed)
 
     small, large = problem(48, 512, 2560, 1), problem(900, 3584, 2560, 2)
     out = torch.empty((48, 512), dtype=torch.bfloat16, device=gpu)
