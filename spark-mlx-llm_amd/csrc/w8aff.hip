@@ -214,19 +214,34 @@ int affine_gemm(const void* x, const uint32_t* w, const void* s, const void* b, 
 
 // Given a workspace, the kernels of affgemm.hip take the call from one row on:
 // they split K over the chip, where the kernel here walks it in one chain
-// (bf16, us per call, here -> there: 1 row of 3584 x 2560 G64 54 -> 18, of
-// 2560 x 4096 G32 182 -> 21, of 131072 x 2560 216 -> 136; 32 rows 66 -> 19,
-// 200 -> 22, 281 -> 142). The kernel here serves calls without a workspace.
-static bool w8_affine_gemm(int64_t M) { return M >= env_int("SPARKQ_W8AFF_GEMM_FROM", 1); }
+// (bf16, us per call, here -> there: 1 row of 3584 x 2560 G64 54 -> 20, of
+// 2560 x 4096 G32 182 -> 20, of 131072 x 2560 209 -> 120; 32 rows 66 -> 20,
+// 199 -> 20, 281 -> 142). A chain of few steps (64 k, 32 at G32) is shorter than
+// their second launch, as long as its tiles of 32 x 128 take few rounds. GPU us
+// here / there, G64: K = 64 (one step) 1 x 2560 4.0 / 7.8, 2048 x 2560 (5 tiles
+// per CU) 16.5 / 20.1, 2048 x 19456 87 / 80; K = 192 (three) 1 x 19456 6.1 / 9.6,
+// 128 x 9728 (1.2 per CU) 11.8 / 13.2, 2048 x 2560 26.6 / 23.1; K = 320 (five)
+// 1 x 32768 8.3 / 11.3, 256 x 2560 11.7 / 14.2, 128 x 9728 16.1 / 14.7; K = 384
+// 64 x 2560 13.5 / 14.2, 16 x 4096 11.6 / 11.3; K = 512 17.0 / 15.5, 14.6 / 12.5.
+// G32: K = 160 (five) 256 x 2560 11.7 / 13.9, 512 x 2560 16.0 / 14.2; K = 256
+// 64 x 2560 16.5 / 14.2. The kernel here also serves calls without a workspace.
+static bool w8_affine_gemm(int64_t M, int64_t N, int64_t K, int G) {
+  const int64_t from = env_int("SPARKQ_W8AFF_GEMM_FROM", -1);
+  if (from >= 0) return M >= from;
+  if (env_int("SPARKQ_AFFG_S", 0) > 0) return true;
+  const int64_t steps = K / (G == 32 ? 32 : 64), tiles = cdiv(M, 32) * cdiv(N, 128);
+  const int64_t rounds = steps <= 1 ? 6 : steps <= 3 ? 2 : steps <= 5 ? 1 : 0;
+  return tiles > rounds * device_cus();
+}
 
 size_t w8_affine_workspace(int64_t M, int64_t N, int64_t K, int G) {
-  return w8_affine_gemm(M) ? affine_gemm_workspace(M, N, K, G) : 0;
+  return w8_affine_gemm(M, N, K, G) ? affine_gemm_workspace(M, N, K, G) : 0;
 }
 
 int w8_affine_linear(const void* x, const uint32_t* w, const void* s, const void* b, void* y,
                      int64_t M, int64_t N, int64_t K, int G, int xdt, int sdt, int ydt, void* ws,
                      size_t wsb, hipStream_t st) {
-  if (ws != nullptr && w8_affine_gemm(M)) {
+  if (ws != nullptr && w8_affine_gemm(M, N, K, G)) {
     const size_t need = w8_affine_workspace(M, N, K, G);
     if (wsb < need)
       return set_error(SPARKQ_ERR_WORKSPACE,

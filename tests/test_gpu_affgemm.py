@@ -106,3 +106,22 @@ def test_error_over_long_rows(gpu, bits, m, n, k, g, dtype, sdtype, s, mean, mon
     bound = (2 * k / g) ** 0.5 * 2.0 ** -24
     print(f"rel {rel:.2e} bound {bound:.2e}", flush=True)
     assert rel <= bound
+
+
+@pytest.mark.parametrize("m,n,k,g", [(1, 130, 64, 64), (33, 200, 320, 64), (40, 130, 96, 32),
+                                     (2, 300, 256, 128), (257, 4096, 320, 64), (5, 70, 384, 64)])
+def test_w8_short_rows_on_both_kernels(gpu, m, n, k, g, monkeypatch):
+    """Around the rule that keeps short rows in one launch: the planned kernel
+    and each of the two agree with the oracle."""
+    import sparkq
+
+    print(f"[case] affgemm w8 short m={m} n={n} k={k} g={g}", flush=True)
+    x, words, sc, b = _problem(m, n, k, g, o.BF16, o.F32, seed=m + n)
+    args = (up16(x, o.BF16, gpu), up32(words, gpu), _dev_scales(sc, o.F32, gpu),
+            _dev_scales(b, o.F32, gpu))
+    ref = o.w8_affine_matmul(x, words, sc, b, g, o.BF16, o.F32)
+    for route in (None, "0", "1000000"):
+        if route is not None:
+            monkeypatch.setenv("SPARKQ_W8AFF_GEMM_FROM", route)
+        y = sparkq.affine_quantized_matmul(*args, group_size=g, bits=8)
+        assert rel_l2(y.cpu().numpy(), ref) <= 1e-6, route
