@@ -1276,8 +1276,7 @@ static bool use_rows_sync(int64_t M, int64_t K, int xdt) {
 // 128 bytes of every row of both operands, staged through LDS (double
 // buffered; 128-byte rows whose 16-byte chunks are swizzled by the row, so
 // the 32 rows a fragment read touches at one chunk index fall on distinct
-// banks); the loads of step s+2 go out before the MFMAs of step s (at 128-row
-// tiles within 2% of one step ahead; small grids wait for their loads). Lane
+// banks); the loads of step s+PD go out before the MFMAs of step s. Lane
 // (l % 32, l / 32) of a fragment holds bytes 16 * (l / 32) .. +15 of row
 // l % 32 of a 32-k sub-step, for activations and weights alike. Grids with
 // fewer tiles than CUs split K into S pieces: each piece stores
@@ -1298,7 +1297,7 @@ __device__ __forceinline__ uint32_t i8_tile_off(int row, int kc) {
   return (uint32_t)(row * 128 + ((kc ^ ((t ^ (t >> 3)) & 7)) << 4));
 }
 
-template <int FR>
+template <int FR, int PD>
 __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
   constexpr int BM = 64 * FR, BN = BM, TB = (BM + BN) * kI8GK;  // bytes per stage
   __shared__ __attribute__((aligned(16))) unsigned char lds[2 * TB];
@@ -1345,12 +1344,14 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
     goff[i] = (uint32_t)(row * K + kc * 16);
     loff[i] = i8_tile_off(row, kc);
   }
-  // register set t holds the loads of the steps of parity t; past the last
-  // step they go to an out-of-range offset (zeros), so that no branch splits
-  // the wait counts
-  u32x4_t va[2][CH], vb[2][CH];
+  // Register set t holds the loads of the steps of parity t (PD = 1: one set).
+  // Two steps ahead, the loads past the last step go to an out-of-range offset
+  // (zeros). The compiler makes branches of that for some of them, whose joins
+  // wait for the loads just issued: part of a step's loads have one step to
+  // arrive, not two.
+  u32x4_t va[PD][CH], vb[PD][CH];
   auto load = [&](int step, int set) {
-    const bool live = step < s_end;
+    const bool live = PD == 1 || step < s_end;
     const int k0 = live ? step * kI8GK : 0;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
@@ -1359,12 +1360,12 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
       vb[set][i] = __builtin_bit_cast(u32x4_t, __builtin_amdgcn_raw_buffer_load_b128(rb, o, k0, 0));
     }
   };
-  auto stage = [&](int buf) {
+  auto stage = [&](int buf, int set) {
     unsigned char* base = lds + buf * TB;
 #pragma unroll
     for (int i = 0; i < CH; ++i) {
-      *reinterpret_cast<u32x4_t*>(base + loff[i]) = va[buf][i];
-      *reinterpret_cast<u32x4_t*>(base + BM * kI8GK + loff[i]) = vb[buf][i];
+      *reinterpret_cast<u32x4_t*>(base + loff[i]) = va[set][i];
+      *reinterpret_cast<u32x4_t*>(base + BM * kI8GK + loff[i]) = vb[set][i];
     }
   };
 
@@ -1376,10 +1377,7 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
   // fragment rows (a multiple of 32 plus l32: the swizzle's t is l32)
   const int ar0 = wm * 32 * FR + l32, br0 = wn * 32 * FR + l32;
 
-  auto body = [&](int step, auto curc) {
-    constexpr int cur = decltype(curc)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    load(step + 2, cur);
+  auto multiply = [&](int cur) {
     const unsigned char* base = lds + cur * TB;
 #pragma unroll
     for (int ss = 0; ss < 4; ++ss) {
@@ -1396,23 +1394,45 @@ __global__ __launch_bounds__(256, 2) void i8_gemm_kernel(I8Args a) {
 #pragma unroll
         for (int y = 0; y < FR; ++y) acc[x][y] = mfma_i8(af[x], bf[y], acc[x][y]);
     }
-    stage(cur ^ 1);  // (last read in the step before, behind its barrier)
-    __syncthreads();
   };
-  if (s_begin < s_end) {
-    load(s_begin, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    load(s_begin + 1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    stage(0);
-    __syncthreads();
+  if constexpr (PD == 1) {
+    if (s_begin < s_end) {
+      load(s_begin, 0);
+      stage(0, 0);
+      __syncthreads();
+    }
+    for (int step = s_begin; step < s_end; ++step) {
+      const int cur = (step - s_begin) & 1;
+      const bool more = step + 1 < s_end;
+      if (more) load(step + 1, 0);
+      multiply(cur);
+      if (more) stage(cur ^ 1, 0);
+      __syncthreads();
+    }
+  } else {
+    auto body = [&](int step, auto curc) {
+      constexpr int cur = decltype(curc)::value;
+      __builtin_amdgcn_sched_barrier(0);
+      load(step + 2, cur);
+      multiply(cur);
+      stage(cur ^ 1, cur ^ 1);  // (last read in the step before, behind its barrier)
+      __syncthreads();
+    };
+    if (s_begin < s_end) {
+      load(s_begin, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      load(s_begin + 1, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      stage(0, 0);
+      __syncthreads();
+    }
+    int step = s_begin;
+    for (; step + 2 <= s_end; step += 2) {
+      body(step, std::integral_constant<int, 0>{});
+      body(step + 1, std::integral_constant<int, 1>{});
+    }
+    if (step < s_end) body(step, std::integral_constant<int, 0>{});
   }
-  int step = s_begin;
-  for (; step + 2 <= s_end; step += 2) {
-    body(step, std::integral_constant<int, 0>{});
-    body(step + 1, std::integral_constant<int, 1>{});
-  }
-  if (step < s_end) body(step, std::integral_constant<int, 0>{});
 
   if (S > 1) {
     // this piece's tile: chunk c (16 bytes) of every thread at (c * 256 + tid) * 16
@@ -1725,7 +1745,7 @@ static I8Plan plan_i8(int64_t M, int64_t N, int64_t K) {
 // least eight steps (tiles within the counter block).
 struct I8GemmPlan {
   bool ok;
-  int FR, tiles_n, tiles, S, full;
+  int FR, PD, tiles_n, tiles, S, full;
   size_t part_bytes;
 };
 
@@ -1769,6 +1789,12 @@ static I8GemmPlan plan_i8_gemm(int64_t M, int64_t N, int64_t K) {
     S = std::min<int64_t>(env_int("SPARKQ_I8_GEMM_SPLITS", 1), K / kI8GK);
     full = 0;
   }
+  // Loads two steps ahead, which small tiles wait for most; the second step's
+  // start and the two past the end cost more than they save on short rows in
+  // less than two rounds of large tiles. One / two ahead, us: 1700 x 2560 x 2560
+  // 23.4 / 25.1, 2048 x 2560 x 2560 24.4 / 25.6, 1700 x 2560 x 1536 19.6 / 20.3;
+  // 1700 x 2560 x 4096 30.2 / 29.3, 2048 x 9728 x 2560 (five rounds) 72.6 / 70.7.
+  p.PD = p.FR == 2 && tiles < 2 * cus && K / kI8GK < 32 ? 1 : 2;
   p.tiles_n = (int)tn;
   p.tiles = (int)tiles;
   p.S = (int)std::max<int64_t>(S, 1);
@@ -1807,9 +1833,11 @@ static int launch_i8_gemm(I8Args args, const I8GemmPlan& p, hipStream_t st) {
   args.full = p.full;
   const dim3 grid((unsigned)(p.full + (p.tiles - p.full) * p.S));
   if (p.FR == 1)
-    hipLaunchKernelGGL(i8_gemm_kernel<1>, grid, dim3(256), 0, st, args);
+    hipLaunchKernelGGL((i8_gemm_kernel<1, 2>), grid, dim3(256), 0, st, args);
+  else if (p.PD == 1)
+    hipLaunchKernelGGL((i8_gemm_kernel<2, 1>), grid, dim3(256), 0, st, args);
   else
-    hipLaunchKernelGGL(i8_gemm_kernel<2>, grid, dim3(256), 0, st, args);
+    hipLaunchKernelGGL((i8_gemm_kernel<2, 2>), grid, dim3(256), 0, st, args);
   return check_launch("i8_gemm_kernel");
 }
 

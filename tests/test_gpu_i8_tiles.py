@@ -37,3 +37,17 @@ def test_i8_planned_exact(gpu, m, n, k):
     a, b = (torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int8) for r in (m, n))
     y = sparkq.int8_matmul_int32(a.to(gpu), b.to(gpu)).cpu()
     assert torch.equal(y.double(), a.double() @ b.double().T)
+
+
+@pytest.mark.parametrize("k", [128, 256, 384, 3968, 4096])
+def test_i8_large_tiles_short_and_long_rows(gpu, k):
+    """128-row tiles with loads one step ahead (fewer than 32 steps of 128 in
+    less than two rounds) and two, down to a single step."""
+    import sparkq
+
+    m, n = 2100, 2050
+    print(f"[case] i8 steps ahead k={k}", flush=True)
+    gen = torch.Generator().manual_seed(k)
+    a, b = (torch.randint(-128, 128, (r, k), generator=gen, dtype=torch.int8) for r in (m, n))
+    y = sparkq.int8_matmul_int32(a.to(gpu), b.to(gpu)).cpu()
+    assert torch.equal(y.double(), a.double() @ b.double().T)
