@@ -1,6 +1,7 @@
 """The division of the 16-bit gelu by 181/128 against the product with its
 fp32 reciprocal, over every finite gate of both 16-bit types: the same 16 bits
-after rounding, as the comment at gelu_mul argues."""
+after rounding, as the comment at gelu_mul argues. This checks the argument in
+numpy; test_gpu_layer_chunks.py runs the kernels over the same gates."""
 
 import numpy as np
 import pytest

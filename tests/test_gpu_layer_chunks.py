@@ -86,3 +86,40 @@ def test_gelu_chunks(gpu, m, inter):
         g16, u16 = (_plain(nrm, t, g, dtype, gpu) for t in (gate, up))
         assert np.array_equal(act, o.gelu_mul16(g16, u16, dtype))
         assert np.array_equal(out, o.add16(hid, _plain(act, down, g, dtype, gpu), dtype))
+
+
+@pytest.mark.parametrize("m", [1, 5, 33])
+def test_gelu_over_every_gate(gpu, m):
+    """act of the FFN over every finite 16-bit gate (the division by 181/128
+    is a product with its reciprocal in the kernels, and a division in the
+    oracle), bit for bit, as the fused decode, the decode and the prefill
+    projections feed it. Weight rows of scale 0 whose bias is the gate, and
+    normed rows that are 1 once and 0 elsewhere, make the gates."""
+    import sparkq
+    from test_gpu_layer import _dev, _plain
+
+    k, inter, g = 64, 65536, 64
+    print(f"[case] every gate m={m}", flush=True)
+    for dtype in (o.BF16, o.F16):
+        bits = np.arange(inter, dtype=np.uint16)
+        bits = np.where(np.isfinite(o.bits_to_f32(bits, dtype)), bits, 0).astype(np.uint16)
+        one = o.round16(np.ones(1, np.float32), dtype)[0]
+        codes, zero = np.zeros((inter, k // 8), np.uint32), np.zeros((inter, 1), np.uint16)
+        gate = (codes, zero, bits[:, None].copy())
+        up = (codes, zero, np.full((inter, 1), one, np.uint16))
+        down = (np.zeros((k, inter // 8), np.uint32), np.zeros((k, inter // g), np.uint16),
+                np.zeros((k, inter // g), np.uint16))
+        x, nw = np.full((m, k), one, np.uint16), np.zeros(k, np.uint16)
+        nw[0] = one
+        zeros = up16(np.zeros((m, k), np.uint16), dtype, gpu)
+        _, _, nrm, act = sparkq.fused_ffn(
+            up16(x, dtype, gpu), zeros, up16(nw, dtype, gpu), 0.0, _dev(gate, gpu, dtype),
+            _dev(up, gpu, dtype), _dev(down, gpu, dtype), group_size=g, return_intermediates=True)
+        rows = np.tile(nw, (m, 1))
+        g16, u16 = (_plain(rows, t, g, dtype, gpu) for t in (gate, up))
+        assert (u16 == one).all()
+        # (the sum with the scale's zero makes -0 a +0)
+        for row in g16:
+            assert np.array_equal(row, np.where(bits == 0x8000, 0, bits))
+        got, ref = down16(act), o.gelu_mul16(g16, u16, dtype)
+        assert np.array_equal(got, ref), int((got != ref).sum())
