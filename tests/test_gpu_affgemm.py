@@ -120,7 +120,7 @@ def test_w8_short_rows_on_both_kernels(gpu, m, n, k, g, monkeypatch):
     args = (up16(x, o.BF16, gpu), up32(words, gpu), _dev_scales(sc, o.F32, gpu),
             _dev_scales(b, o.F32, gpu))
     ref = o.w8_affine_matmul(x, words, sc, b, g, o.BF16, o.F32)
-    for route in (None, "0", "1000000"):
+    for route in (None, "1", "1000000"):
         if route is not None:
             monkeypatch.setenv("SPARKQ_W8AFF_GEMM_FROM", route)
         y = sparkq.affine_quantized_matmul(*args, group_size=g, bits=8)
