@@ -949,6 +949,8 @@ def main():
         tr = gemm_trace()
         if "gate_up_m2048_kernel_us" in tr:
             ku = tr["gate_up_m2048_kernel_us"]
+            # (a profiled run of its own, not this one)
+            roofline_gemm["kernel_only_source"] = os.path.relpath(GEMM_TRACE_FILE, ROOT)
             roofline_gemm["kernel_only_avg_us_rocprof"] = ku
             roofline_gemm["kernel_only_TFLOP/s_rocprof"] = round(flop / ku / 1e6, 1)
             roofline_gemm["kernel_only_frac_rocprof"] = round(flop / ku / 1e6 / BF16_PEAK_TFLOPS, 4)

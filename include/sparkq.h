@@ -128,8 +128,10 @@ int sparkq_w4a16_linear(const void* x, const uint32_t* w, const void* scales,
  * arrays change (spark_mlx_llm/ops/linear.py:260-268, built by
  * prepare_w4a16_nax4, X/spark_mlx_ext/w4a16_multirow.py:169-222). It holds
  * the weight half of the bf16 GEMM prologue: per-row power-of-two shifted
- * fp16 scales [N,K/G], the row shifts [N] and the bias slots [N,3K/G
- * padded to 16] (b + 8s split into bf16 pairs). Only bfloat16 scales and
+ * fp16 scales [K/G,N], the row shifts [N] and the bias slots [N,3K/G
+ * padded to 16] (b + 8s split into bf16 pairs). The layout is this library's
+ * own and may differ in another version: make the buffer anew at load time,
+ * do not store it. Only bfloat16 scales and
  * biases have a prepared form. sparkq_w4a16_prepared_bytes gives its size
  * (0 for an unsupported group size); the buffer must be 256-byte aligned.
  * Reads scales and biases only; never allocates. */

@@ -30,10 +30,12 @@
 // tiles do not fill the chip, pieces of K go to workgroups of their own and
 // affine_sum_kernel adds their fp32 sums in order.
 //
-// What bounds it: the latency of the units' chain, at many tiles the turns that
-// LDS reads, the VALU and the MFMA take (about 0.25 us a unit each). 64
-// columns per wave, which would halve the LDS reads, have no registers for it
-// and measured 0-20% slower. 4-bit instances fit three workgroups on a CU, 8-bit
+// What bounds it: the latency of the units' chain and the decode beside it: at
+// one workgroup per CU (8-bit 512 x 3584 x 2560) a unit takes 1.7 us, waves wait
+// 35% of the time, issue VALU 31%, and MFMAs are busy 12%; at two (4-bit 333 x
+// 2560 x 9728) 1.8 us, 32%, 26% and 21%. Of the calls' time 8 to 14 us go to the
+// prologue and the sum of the pieces. 64 columns per wave, which would halve
+// the LDS reads, have no registers for it and measured 0-20% slower. 4-bit instances fit three workgroups on a CU, 8-bit
 // ones two. Per call, against the kernels this replaced: fp16 4-bit 333 x 2560 x
 // 9728 G128 234 -> 45 us, 512 x 3584 x 2560 G64 68 -> 34, 2048 x 19456 x 2560
 // G64 371 -> 314 (650 TFLOP/s); bf16 8-bit 512 x 3584 x 2560 G64 104 -> 39,
@@ -335,13 +337,14 @@ struct AffLayout {
   size_t st, bt, xs, part, bytes;
 };
 // Pieces of K, at most 8 and of at least three units: the number that
-// minimises an estimate in us. A unit takes about 1 us in a workgroup that has
-// a CU to itself and 1.5 us where two share one, two is what a CU holds, and
-// pieces cost a launch and their partials' round trip. Measured per call in
-// 1, 2, 3, 4, 6, 8 pieces: fp16 4-bit 333 x 2560 x 9728 G128 87, 56, 56, 48,
-// 47, 51 us; 512 x 3584 x 2560 G64 40, 40, 39, 42, 45, 47; 2048 x 2560 x 9728
-// 194, 181, 189, 186, 197, 210; bf16 8-bit 333 x 2560 x 9728 115, 70, 65, 54,
-// 62, 61; 64 x 3584 x 2560 37, 25, 22, 21, 20, 21.
+// minimises an estimate. Its unit times (1 in a workgroup that has a CU to
+// itself, 1.5 where two share one) are below the traced ones (1.7 and 1.8 us),
+// and order the pieces as measured beside what these cost, a launch and their
+// partials' round trip. Us per call in 1, 2, 3, 4, 6, 8 pieces (its choice in
+// brackets): fp16 4-bit 333 x 2560 x 9728 G128 79, 50, 48, [42], 43, 46; 512 x
+// 3584 x 2560 G64 [33], 36, 36, 38, 42, 43; 2048 x 2560 x 9728 G128 157, 151, 161,
+// [159], 167, 177; bf16 8-bit 333 x 2560 x 9728 G64 98, 59, 61, [51], 55, 57; 64 x
+// 3584 x 2560 33, 23, 20, 19, 18, 19 [five: 18]; 1 x 2560 x 4096 G32 52, 33, 26, 22, 20, [18].
 int aff_pieces(int64_t M, int64_t N, int64_t K) {
   const int64_t cus = device_cus(), units = cdiv(K, kAffBK);
   if (const int64_t s = env_int("SPARKQ_AFFG_S", 0); s > 0)

@@ -24,15 +24,19 @@
 // weights are the second product's operand where the first one left them.
 //
 // What bounds it: the VALU (per weight: the exponential, per group the scaling
-// and the split, 13 operations) beside four MFMAs' worth of products. Two
-// waves per SIMD overlap the two; head dim 256 has registers for one. Against
-// the vector kernel (one workgroup per query row, whose LDS reads bound it),
-// in us with the append's time left out: 32/8 heads of 128, L = 512 over N =
-// 4096 causal, 4-bit G64 7400 -> 137, 8-bit G32 10650 -> 190; 16/4 heads of
-// 256, 8-bit G32 10520 -> 254; 12/4 heads of 96, L = 300 of N = 1000, 2-bit
-// 476 -> 34; one query token with a mask array over N = 4096 68 -> 16, 12/4
-// heads of 96 over N = 300 52 -> 15. Relative error of the fp32 output against
-// float64: 2e-7 .. 8e-7 (vector kernel 5e-7 .. 1.2e-6).
+// and the split, 13 operations; ten VALU instructions per MFMA in all). Two
+// waves per SIMD overlap the two (head dim 128 G64, L = 512 over N = 4096: waves
+// issue 51% of their time, MFMAs are busy 24%); head dim 256 has registers for
+// one wave per SIMD. Registers spill at head dim 128 G32 (35 to 41 a lane), 256
+// G32 (64) and 256 G64 (6). Additive masks are read one value at a time and
+// cost half as much again (108 -> 171 us; boolean ones 134). Us per call with
+// the merge, against the vector kernel (one workgroup per query row, whose LDS
+// reads bound it): 32/8 heads of 128, L = 512 over N = 4096 causal, 4-bit G64
+// 7400 -> 108, 8-bit G32 10650 -> 165; 16/4 heads of 256, 8-bit G32 10520 -> 241;
+// 12/4 heads of 96, L = 300 of N = 1000, 2-bit 476 -> 30; one query token with a
+// boolean mask array over N = 4096 68 -> 16, 12/4 heads of 96 over N = 300 52 ->
+// 14. Relative error of the fp32 output against float64: 2e-7 .. 8e-7 (vector
+// kernel 5e-7 .. 1.2e-6).
 #include <algorithm>
 #include <cfloat>
 
@@ -479,7 +483,10 @@ void launch_stage_g(const GenSdpaArgs& a, dim3 grid, hipStream_t st) {
 
 // Context splits: two workgroups per CU over the row tiles (two waves per SIMD,
 // so that one's softmax overlaps the other's products), at least two 32-token
-// blocks each.
+// blocks each. Us for 256 / 512 / 768 workgroups: 32/8 heads of 128, L = 512
+// over N = 4096 155 / 108 / 121. Head dim 256, where a CU holds one workgroup,
+// takes two rounds of them: 16/4 heads, L = 512 over N = 2048 129 / 139 / 166, over
+// 512 43 / 51 / 51, L = 100 over 4096 62 / 72 / 91.
 int sdpa_stage_splits(int64_t B, int64_t Hq, int64_t Hkv, int64_t L, int64_t N) {
   const int64_t items = cdiv(L * (Hq / Hkv), kStageRows) * B * Hkv;
   const int64_t S = std::min<int64_t>(cdiv(512, items), std::max<int64_t>(N / 64, 1));
