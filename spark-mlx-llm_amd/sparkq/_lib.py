@@ -107,9 +107,12 @@ def lib():
     return _LIB
 
 
+_DTYPE_CODES = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
+
+
 def dtype_code(dtype: torch.dtype) -> int:
     try:
-        return {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}[dtype]
+        return _DTYPE_CODES[dtype]
     except KeyError:
         raise ValueError(f"unsupported floating dtype {dtype}") from None
 
